@@ -86,6 +86,110 @@ __global__ void q4_gemv_kernel(const uint32_t* __restrict__ packed,
   if (lane == 0) y[row] = acc;
 }
 
+// nib_dot8 of a word by the two in-place masks of nib_dot32, four products to
+// a chain.
+__device__ __forceinline__ float nib_dot8_masks(uint32_t w, const float* x) {
+  const uint32_t t = w >> 8;
+  const uint32_t p0 = w & 0x000F000Fu, p1 = w & 0x00F000F0u;
+  const uint32_t p2 = t & 0x000F000Fu, p3 = t & 0x00F000F0u;
+  float a = fmaf(f16_lo(p0), x[0], opaque_zero());
+  float b = fmaf(f16_lo(p1), x[1], opaque_zero());
+  a = fmaf(f16_lo(p2), x[2], a);
+  b = fmaf(f16_lo(p3), x[3], b);
+  a = fmaf(f16_hi(p0), x[4], a);
+  b = fmaf(f16_hi(p1), x[5], b);
+  a = fmaf(f16_hi(p2), x[6], a);
+  b = fmaf(f16_hi(p3), x[7], b);
+  return fmaf(b, kTwo20, a * kTwo24);
+}
+
+// The same GEMV for rows of whole 16-byte chunks (32 columns, each inside one
+// group): LPR lanes share a row, a lane takes chunks c, c + LPR, ..., and a
+// wavefront keeps RPW x (64 / LPR) rows in flight. x is staged in LDS, LPR
+// chunks at a time and 36 floats apart so that the lanes' 16-byte reads
+// spread over the banks, and read back once for all of a wavefront's rows.
+// Bound by the latency of one round of loads up to a few MB of weights (a
+// launch that does nothing takes 2.3 µs), then by the loads in flight. µs a
+// launch, word-wise kernel above / this one, kernel trace: 640 x 2048 f32
+// metadata 3.96 / 2.96, 4096 x 2048 f32 5.68 / 4.32, 1000 x 4992 bf16 8.28 /
+// 5.44, 16384 x 2048 bf16 12.5 / 7.8, 16384 x 5120 f32 27.6 / 16.7 (3.1 TB/s).
+// Loading the next chunks before multiplying these measured 7.0 and 16.3 at
+// the two largest, and spilled at one row per wavefront.
+template <int META, int LPR, int RPW>
+__global__ __launch_bounds__(256) void q4_gemv_chunks_kernel(const uint32_t* __restrict__ packed,
+                                                             const void* __restrict__ scales,
+                                                             const void* __restrict__ biases, uint32_t out_dim,
+                                                             uint32_t packed_cols, uint32_t group,
+                                                             const float* __restrict__ x, float* __restrict__ y) {
+  constexpr uint32_t kStep = kWave / LPR;  // rows side by side in a wavefront
+  constexpr uint32_t kStride = 36;
+  __shared__ __align__(16) float xs[LPR * kStride];
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t c0 = lane % LPR;
+  const uint32_t r0 = (blockIdx.x * 4u + threadIdx.x / kWave) * (kStep * RPW) + lane / LPR;
+  const uint32_t nch = packed_cols / 4u, groups = packed_cols * 8u / group;
+  float acc[RPW];
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) acc[i] = 0.0f;
+  for (uint32_t cb = 0; cb < nch; cb += LPR) {
+    // Lanes past the row's end and rows past the last read the last chunk or
+    // row again; their values are not added, or not stored.
+    const uint32_t cc = cb + c0 < nch ? cb + c0 : nch - 1u;
+    const uint32_t g = cc * 32u / group;
+    uint4 q[RPW];
+    uint32_t sb[RPW], bb[RPW];
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const uint32_t r = r0 + i * kStep < out_dim ? r0 + i * kStep : out_dim - 1u;
+      q[i] = ldg16(packed + (static_cast<size_t>(r) * nch + cc) * 4u);
+      const size_t gi = static_cast<size_t>(r) * groups + g;
+      sb[i] = meta_bits<META>(scales, gi);
+      bb[i] = meta_bits<META>(biases, gi);
+    }
+    if (cb > 0u) __syncthreads();  // the previous chunks are read
+    const float4* x4 = reinterpret_cast<const float4*>(x) + cb * 8u;
+    const uint32_t n4 = (nch - cb) * 8u;
+    for (uint32_t f = threadIdx.x; f < LPR * 8u; f += 256u)
+      *reinterpret_cast<float4*>(xs + (f / 8u) * kStride + (f % 8u) * 4u) =
+          f < n4 ? x4[f] : make_float4(0.f, 0.f, 0.f, 0.f);
+    __syncthreads();
+    float xr[32];
+    const float4* xl = reinterpret_cast<const float4*>(xs + c0 * kStride);
+    float xsum[4];  // of each word's columns
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const float4 f = xl[v];
+      xr[4 * v] = f.x; xr[4 * v + 1] = f.y; xr[4 * v + 2] = f.z; xr[4 * v + 3] = f.w;
+      const float s4 = (f.x + f.y) + (f.z + f.w);
+      xsum[v / 2] = v % 2 ? xsum[v / 2] + s4 : s4;
+    }
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      // Scale and bias per word, as the word-wise kernel adds them: their
+      // products largely cancel, and summed over 32 columns first they leave
+      // a larger error.
+      const float sc = meta_widen<META>(sb[i]), bi = meta_widen<META>(bb[i]);
+      const uint32_t w4[4] = {q[i].x, q[i].y, q[i].z, q[i].w};
+      float v = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v += sc * nib_dot8_masks(w4[k], xr + 8 * k) + bi * xsum[k];
+      acc[i] += cb + c0 < nch ? v : 0.0f;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) {
+    float v = acc[i];
+    if constexpr (LPR == 64)
+      v = wave_sum(v);
+    else if constexpr (LPR == 32)
+      v = group_sum(v, 32);
+    else
+      v = row_sum<LPR>(v);
+    const uint32_t r = r0 + i * kStep;
+    if (c0 == 0u && r < out_dim) y[r] = v;
+  }
+}
+
 __global__ void unpack_kernel(const uint32_t* __restrict__ packed, size_t words,
                               uint8_t* __restrict__ out) {
   const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
@@ -240,6 +344,43 @@ __global__ __launch_bounds__(kQuantThreads) void quant_pack_kernel(
   }
 }
 
+// Below this many packed words the word-wise kernel is as fast: its loads
+// leave at once, without the barrier (µs, word-wise / chunks: 256 x 512 and
+// 512 x 512 2.32 / 2.52, 2048 x 512 2.76 / 2.72; 640 x 2048 3.96 / 2.96).
+constexpr uint64_t kGemvChunksMinWords = 1u << 17;
+
+template <int META, int LPR, int RPW>
+int launch_gemv_chunks(const osmd_q4_proj& p, const float* x, float* y, hipStream_t st) {
+  constexpr uint32_t rows = 4u * (kWave / LPR) * RPW;  // per workgroup
+  q4_gemv_chunks_kernel<META, LPR, RPW><<<(p.out_dim + rows - 1u) / rows, 256, 0, st>>>(
+      p.packed, p.scales, p.biases, p.out_dim, p.packed_cols, p.group, x, y);
+  return launch_status();
+}
+
+// Rows per wavefront: as many as leave 2,048 wavefronts, two to a SIMD.
+template <int META, int LPR>
+int launch_gemv_lanes(const osmd_q4_proj& p, const float* x, float* y, hipStream_t st) {
+  const uint64_t waves = (static_cast<uint64_t>(p.out_dim) * LPR + kWave - 1u) / kWave;
+  if (waves >= 4u * 2048u) return launch_gemv_chunks<META, LPR, 4>(p, x, y, st);
+  if (waves >= 2u * 2048u) return launch_gemv_chunks<META, LPR, 2>(p, x, y, st);
+  return launch_gemv_chunks<META, LPR, 1>(p, x, y, st);
+}
+
+template <int META>
+int launch_gemv(const osmd_q4_proj& p, const float* x, float* y, hipStream_t st) {
+  const uint64_t words = static_cast<uint64_t>(p.out_dim) * p.packed_cols;
+  if (words >= kGemvChunksMinWords && p.packed_cols % 4u == 0u && p.group % 32u == 0u &&
+      ((reinterpret_cast<uintptr_t>(p.packed) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0u) {
+    const uint32_t nch = p.packed_cols / 4u;
+    if (nch <= 16u) return launch_gemv_lanes<META, 16>(p, x, y, st);
+    if (nch <= 32u) return launch_gemv_lanes<META, 32>(p, x, y, st);
+    return launch_gemv_lanes<META, 64>(p, x, y, st);
+  }
+  q4_gemv_kernel<META><<<(p.out_dim + 3u) / 4u, 256, 0, st>>>(p.packed, p.scales, p.biases, p.out_dim, p.packed_cols,
+                                                             p.group, x, y);
+  return launch_status();
+}
+
 }  // namespace
 
 extern "C" {
@@ -264,19 +405,11 @@ int osmd_q4_dequant(const osmd_q4_proj* p, float* out, osmd_stream s) {
 
 int osmd_q4_gemv(const osmd_q4_proj* p, const float* x, float* y, osmd_stream s) {
   const hipStream_t st = static_cast<hipStream_t>(s);
-  const unsigned grid = (p->out_dim + 3u) / 4u;  // 4 waves (rows) per block
   switch (p->meta_dtype) {
-    case OSM_META_F32:
-      q4_gemv_kernel<OSM_META_F32><<<grid, 256, 0, st>>>(p->packed, p->scales, p->biases, p->out_dim, p->packed_cols, p->group, x, y);
-      break;
-    case OSM_META_F16:
-      q4_gemv_kernel<OSM_META_F16><<<grid, 256, 0, st>>>(p->packed, p->scales, p->biases, p->out_dim, p->packed_cols, p->group, x, y);
-      break;
-    default:
-      q4_gemv_kernel<OSM_META_BF16><<<grid, 256, 0, st>>>(p->packed, p->scales, p->biases, p->out_dim, p->packed_cols, p->group, x, y);
-      break;
+    case OSM_META_F32: return launch_gemv<OSM_META_F32>(*p, x, y, st);
+    case OSM_META_F16: return launch_gemv<OSM_META_F16>(*p, x, y, st);
+    default: return launch_gemv<OSM_META_BF16>(*p, x, y, st);
   }
-  return launch_status();
 }
 
 int osmd_unpack_nibbles(const uint32_t* packed, size_t words, uint8_t* out, osmd_stream s) {
