@@ -90,6 +90,7 @@ struct RouteView {
   const float* logits;                // [B, E]
   const float* bounds;                // [B, E] bound of each logit, or null (no bound: exact path)
   const float* planes;                // null, or `parts` planes [B][E + 1] of partial sums
+  const float* planes_lo;             // with planes: what their rounding to fp32 left, or null
   const float* bound_planes;          // with planes: [parts][B][E + 1] bound parts, or null
   uint32_t parts, tokens;
   float* logits_out;                  // [B, E]  with planes: the summed logits
@@ -1104,7 +1105,29 @@ __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Se
       const bool bounded = rv.bound_planes != nullptr;
       const float cols = static_cast<float>(D / rv.parts);
       float v, rs = 0.0f;
-      if (rv.parts <= kMaxPlanes) {
+      if (rv.planes_lo != nullptr) {
+        // Planes of fp64 sums: added up in fp64, rounded once.
+        const float* plo = rv.planes_lo + o;
+        double vd = 0.0;
+        for (uint32_t p0 = 0; p0 < rv.parts; p0 += 4u) {
+          float hi[4], lo[4], rb[4];
+#pragma unroll
+          for (uint32_t i = 0; i < 4u; ++i) {
+            const uint32_t part = p0 + i < rv.parts ? p0 + i : p0;  // read again, not added
+            hi[i] = pl[part * ps];
+            lo[i] = plo[part * ps];
+            rb[i] = bounded ? rv.bound_planes[part * ps + o] : 0.0f;
+          }
+#pragma unroll
+          for (uint32_t i = 0; i < 4u; ++i) {
+            if (p0 + i < rv.parts) {
+              rs += rb[i] + cols * fabsf(static_cast<float>(vd));
+              vd += static_cast<double>(hi[i]) + lo[i];
+            }
+          }
+        }
+        v = static_cast<float>(vd);
+      } else if (rv.parts <= kMaxPlanes) {
         // Every plane's loads issued before the first addition.
         float pv[kMaxPlanes], rb[kMaxPlanes];
 #pragma unroll
@@ -1144,9 +1167,16 @@ __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Se
   }
   if (PLANES && rv.planes != nullptr && rv.has_shared && threadIdx.x == 0) {
     const size_t ps = static_cast<size_t>(rv.tokens) * (E + 1u);
-    const float* pl = rv.planes + static_cast<size_t>(t) * (E + 1u) + E;
-    float g = pl[0];
-    for (uint32_t part = 1; part < rv.parts; ++part) g += pl[part * ps];
+    const size_t o = static_cast<size_t>(t) * (E + 1u) + E;
+    float g = rv.planes[o];
+    if (rv.planes_lo != nullptr) {
+      double gd = 0.0;
+      for (uint32_t part = 0; part < rv.parts; ++part)
+        gd += static_cast<double>(rv.planes[o + part * ps]) + rv.planes_lo[o + part * ps];
+      g = static_cast<float>(gd);
+    } else {
+      for (uint32_t part = 1; part < rv.parts; ++part) g += rv.planes[o + part * ps];
+    }
     rv.gate_out[t] = 1.0f / (1.0f + expf(-g));  // reference_ops.cpp:214-216
   }
   select_values<PER, DEEP>(rv, t, p, bnd, tab, out, count, need_p);
@@ -1731,6 +1761,257 @@ __global__ __launch_bounds__(kDownThreads) void down_kernel(DownParams p) {
 
 
 // ---------------------------------------------------------------------------
+// The router of many tokens when it is not bf16 (fp32, f16 or affine q8
+// values): the per-token kernel's fp64 dot products as a GEMM on the fp64
+// matrix cores, v_mfma_f64_16x16x4. As one wavefront per token and router row
+// the 8-bit router of a 512-token pass took 400 µs, more than twice the
+// experts' gate and up GEMM; this takes 48 µs, with the same products (exact
+// in fp64) and the logit rounded once: the same bits. (Three bf16 terms per
+// element on the bf16 cores took 51 µs and came out with 2.8 times the
+// logits' error.)
+//
+// A: lane l holds token l % 16 at k-slot l / 16; B: router row l % 16; D: lane
+// l's values v are token 4 v + l / 16 of row l % 16. A workgroup is 16 tokens
+// x 64 router rows (a wavefront 16 rows) x one range of R = 16 * NB columns.
+// The tokens are staged in LDS in fp32; each wavefront streams its own router
+// rows, lane l the columns 4 (l / 16) .. + 3 of every 16-column block, with
+// the next four blocks in flight while four are multiplied. A block's four MFMAs take
+// those columns one after another, so the running sum is known at every 16th
+// column. The matrix cores' share is 14 µs (64 cycles per MFMA, 540,672 of
+// them over 1,024 SIMDs); the rest is vector work that does not overlap with
+// fp64 MFMAs on its SIMD: conversions to fp64, dequantisation, bounds (ten
+// instructions per MFMA). Two token tiles to a wavefront's router rows
+// measured 53 µs; the rows held in registers for two tiles filled the
+// register file, 123 µs.
+//
+// The launch is one-dimensional and a multiple of 8 long, its items dealt to
+// the XCDs in runs of one K range, as the bf16 router GEMM's are.
+//
+// Each logit plane gets its part of the bound on the distance from the
+// reference's logit (as route_block derives it: u (sum |P_c| + (2 + 4
+// [RMSNorm] + n^2 u) sum |p_c| + |l|), P_c the exact prefix sums). Over a
+// 16-column block that starts at the running sum S_b the prefix sums add up
+// to at most 16 |S_b| + 16 (sum of the block's |p_c|), and sum |p_c| is at
+// most the product of the 32-column norms of row and input. The selection
+// adds R |running sum| for each range after the first and scales by
+// (1 + 2^-9) u.
+// 64 columns of 16 router rows as lane (m, q) multiplies them: block j's
+// columns c + 16 j + 4 q .. + 3 of row m, j < 4. fp32 and f16 are loaded so;
+// affine q8 as the row's 16 bytes at c + 16 q, which the four lanes of a row
+// then exchange (word j of lane q is lane j's word q): one load of 64
+// consecutive bytes per row instead of four of 16, whose addresses bound the
+// pass (80 µs against 48). A word never straddles a
+// group; scales and biases come per block, or once when groups hold whole
+// 64-column runs.
+template <int RD>
+struct Raw64 {
+  uint32_t v[4][RD == OSM_META_F32 ? 4 : RD == OSM_META_F16 ? 2 : 1];
+  uint32_t s[RD == OSM_ROUTER_AFFINE_Q8 ? 4 : 1], b[RD == OSM_ROUTER_AFFINE_Q8 ? 4 : 1];
+};
+// magic = 2^32 / group rounded up: the high product is c / group exactly for
+// c < 2^16 (it exceeds c / group by less than c / 2^32, below 1 / group).
+template <int RD>
+__device__ __forceinline__ void load_raw64(const uint8_t* base, const Q8Row& qr, uint32_t magic, uint32_t c,
+                                           uint32_t q, Raw64<RD>& r) {
+  if constexpr (RD == OSM_ROUTER_AFFINE_Q8) {
+    const uint4 w = ldg16(qr.q + (c + 16u * q) / 4u);
+    r.v[0][0] = w.x;
+    r.v[1][0] = w.y;
+    r.v[2][0] = w.z;
+    r.v[3][0] = w.w;
+    const bool one = qr.group % 64u == 0u;  // wavefront-uniform
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j) {
+      if (j > 0u && one) {
+        r.s[j] = r.s[0];
+        r.b[j] = r.b[0];
+      } else {
+        const uint32_t g = __umulhi(c + 16u * j + 4u * q, magic);
+        r.s[j] = ldg<uint32_t>(qr.s + g);
+        r.b[j] = ldg<uint32_t>(qr.b + g);
+      }
+    }
+  } else {
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j) {
+      const uint32_t cc = c + 16u * j + 4u * q;
+      if constexpr (RD == OSM_META_F16) {
+        const uint2 h = ldg8(base + 2u * cc);
+        r.v[j][0] = h.x;
+        r.v[j][1] = h.y;
+      } else {
+        const uint4 f = ldg16(base + 4u * cc);
+        r.v[j][0] = f.x;
+        r.v[j][1] = f.y;
+        r.v[j][2] = f.z;
+        r.v[j][3] = f.w;
+      }
+    }
+  }
+}
+// The q8 exchange: a 4 x 4 transpose of words over the lanes q = l / 16 of a
+// row. permlane32_swap(a, b) exchanges a of lanes 32-63 with b of lanes 0-31,
+// permlane16_swap a of each odd row of 16 lanes with b of the even row before.
+__device__ __forceinline__ void transpose_q(uint32_t (&v)[4][1]) {
+  auto swap32 = [](uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  };
+  auto swap16 = [](uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  };
+  swap32(v[0][0], v[2][0]);
+  swap32(v[1][0], v[3][0]);
+  swap16(v[0][0], v[1][0]);
+  swap16(v[2][0], v[3][0]);
+}
+template <int RD>
+__device__ __forceinline__ float raw64_get(const Raw64<RD>& r, int j, int i) {
+  if constexpr (RD == OSM_ROUTER_AFFINE_Q8)
+    return dequant_q8(__uint_as_float(r.s[j]), static_cast<float>((r.v[j][0] >> (8 * i)) & 0xFFu),
+                      __uint_as_float(r.b[j]));
+  else if constexpr (RD == OSM_META_F16)
+    return f16_to_f32((r.v[j][i / 2] >> (16 * (i % 2))) & 0xFFFFu);
+  else
+    return __uint_as_float(r.v[j][i]);
+}
+
+template <int RD, int NB, bool XBF16>
+__global__ __launch_bounds__(256) void router_f64_kernel(
+    const void* __restrict__ x, uint32_t T, uint32_t D, const void* __restrict__ router,
+    const void* __restrict__ shared_gate_vec, uint32_t E, uint32_t group, uint32_t rms, float* __restrict__ planes,
+    float* __restrict__ planes_lo, const float* __restrict__ rnorm, const float* __restrict__ xnorm,
+    float* __restrict__ bplanes, uint32_t gx, uint32_t gy, uint32_t gz) {
+  typedef double f64x4 __attribute__((ext_vector_type(4)));
+  constexpr uint32_t R = 16u * NB;
+  constexpr uint32_t RS = R + 4u;  // LDS row stride (floats), padded against bank conflicts
+  constexpr uint32_t kTok = 16u;
+  static_assert(NB % 4 == 0, "whole batches of 64 columns");
+  constexpr uint32_t kNorm4 = R / 128u;  // 32-column norms of a row's range, four at a time (R and D: of 128 columns)
+  __shared__ __align__(16) float xs[kTok][RS];
+  __shared__ __align__(16) float xn[kTok][4u * kNorm4];
+  const uint32_t n8 = gridDim.x / 8u;
+  const uint32_t item = (blockIdx.x % 8u) * n8 + blockIdx.x / 8u;
+  if (item >= gx * gy * gz) return;  // the launch's padding (workgroup-uniform, before any barrier)
+  const uint32_t bx = item % gx, by = (item / gx) % gy, bz = item / (gx * gy);
+  const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const uint32_t m = lane % 16u, q = lane / 16u;
+  const uint32_t k0 = bz * R, t0 = by * kTok;
+  const uint32_t nrows = E + (shared_gate_vec ? 1u : 0u);
+  const uint32_t row = (bx * kRouteWaves + wave) * 16u + m;
+  const uint32_t rr = row < nrows ? row : nrows - 1u;
+  // Row E is the shared-gate vector's only row.
+  const uint8_t* base = nullptr;
+  Q8Row qr{};
+  uint32_t magic = 0u;
+  if constexpr (RD == OSM_ROUTER_AFFINE_Q8) {
+    qr = rr < E ? q8_row(router, E, rr, D, group) : q8_row(shared_gate_vec, 1u, 0u, D, group);
+    magic = 0xFFFFFFFFu / group + 1u;
+  } else {
+    base = static_cast<const uint8_t*>(rr < E ? router : shared_gate_vec) +
+           static_cast<size_t>(rr < E ? rr : 0u) * D * (RD == OSM_META_F32 ? 4u : 2u);
+  }
+  Raw64<RD> next;
+  load_raw64<RD>(base, qr, magic, k0, q, next);
+  // The chunk norms of this lane's row, and (LDS) of the tokens.
+  float4 rn[kNorm4];
+#pragma unroll
+  for (uint32_t c = 0; c < kNorm4; ++c)
+    rn[c] = reinterpret_cast<const float4*>(rnorm + static_cast<size_t>(rr) * (D / 32u) + k0 / 32u)[c];
+  if (tid < kTok * kNorm4) {
+    const uint32_t r = tid / kNorm4, c = tid % kNorm4;
+    reinterpret_cast<float4*>(&xn[r][0])[c] = reinterpret_cast<const float4*>(
+        xnorm + static_cast<size_t>(t0 + r < T ? t0 + r : T - 1u) * (D / 32u) + k0 / 32u)[c];
+  }
+  for (uint32_t i = tid; i < kTok * (R / 4u); i += 256u) {
+    const uint32_t r = i / (R / 4u), c = i % (R / 4u) * 4u;
+    const size_t o = static_cast<size_t>(t0 + r < T ? t0 + r : T - 1u) * D + k0 + c;  // rows past T: the last token
+    float4 v;
+    if constexpr (XBF16) {
+      const uint2 h = ldg8(static_cast<const uint16_t*>(x) + o);
+      v = make_float4(bf16_to_f32(h.x & 0xFFFFu), bf16_to_f32(h.x >> 16), bf16_to_f32(h.y & 0xFFFFu),
+                      bf16_to_f32(h.y >> 16));
+    } else {
+      v = *reinterpret_cast<const float4*>(static_cast<const float*>(x) + o);
+    }
+    *reinterpret_cast<float4*>(&xs[r][c]) = v;
+  }
+  __syncthreads();
+  if ((bx * kRouteWaves + wave) * 16u >= nrows) return;  // a wavefront past the last row, after the only barrier
+  f64x4 acc = {0.0, 0.0, 0.0, 0.0}, sabs = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+  for (uint32_t b0 = 0; b0 < NB; b0 += 4u) {
+    Raw64<RD> cur = next;
+    load_raw64<RD>(base, qr, magic, k0 + 16u * (b0 + 4u < NB ? b0 + 4u : b0), q, next);
+    if constexpr (RD == OSM_ROUTER_AFFINE_Q8) transpose_q(cur.v);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 a = *reinterpret_cast<const float4*>(&xs[m][16u * (b0 + j) + 4u * q]);
+      // The prefix sum at the block's start (zero at the range's).
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sabs[v] += fabs(acc[v]);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, raw64_get<RD>(cur, j, 0), acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, raw64_get<RD>(cur, j, 1), acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a.z, raw64_get<RD>(cur, j, 2), acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a.w, raw64_get<RD>(cur, j, 3), acc, 0, 0, 0);
+    }
+  }
+  const float n = static_cast<float>(D);
+  const float ca = 16.0f + (rms ? 6.0f : 2.0f) + n * n * 0x1p-24f;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const uint32_t t = t0 + 4u * v + q;
+    if (t >= T || row >= nrows) continue;
+    float ap = 0.0f;
+#pragma unroll
+    for (uint32_t c = 0; c < kNorm4; ++c) {
+      const float4 xv = reinterpret_cast<const float4*>(&xn[4u * v + q][0])[c];
+      ap = fmaf(rn[c].x, xv.x, ap);
+      ap = fmaf(rn[c].y, xv.y, ap);
+      ap = fmaf(rn[c].z, xv.z, ap);
+      ap = fmaf(rn[c].w, xv.w, ap);
+    }
+    const size_t o = (static_cast<size_t>(bz) * T + t) * (E + 1u) + row;
+    const float hi = static_cast<float>(acc[v]);
+    planes[o] = hi;
+    planes_lo[o] = static_cast<float>(acc[v] - hi);
+    bplanes[o] = 16.0f * static_cast<float>(sabs[v]) + fabsf(hi) + ca * ap;
+  }
+}
+
+// Norms of a router's 32-column chunks, [rows][D/32] (row E the shared-gate
+// vector), rounded up: a thread per 8 columns, four of them to a chunk.
+template <int RD>
+__global__ __launch_bounds__(256) void router_norms_kernel(const void* __restrict__ router,
+                                                           const void* __restrict__ shared_gate_vec, uint32_t E,
+                                                           uint32_t D, uint32_t group, float* __restrict__ norms) {
+  const uint32_t row = blockIdx.y;
+  const uint32_t wd = blockIdx.x * 256u + threadIdx.x;
+  const bool in = wd < D / 8u;  // D % 32 == 0: a chunk's four words are in or out together
+  const uint32_t c = (in ? wd : 0u) * 8u;
+  Raw8<RD> raw;
+  if constexpr (RD == OSM_ROUTER_AFFINE_Q8)
+    load_q8x8(row < E ? q8_row(router, E, row, D, group) : q8_row(shared_gate_vec, 1u, 0u, D, group), c, raw);
+  else
+    load_raw8<RD>(static_cast<const uint8_t*>(row < E ? router : shared_gate_vec) +
+                      static_cast<size_t>(row < E ? row : 0u) * D * (RD == OSM_META_F32 ? 4u : 2u), c, raw);
+  double sq = 0.0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const double v = raw8_get<RD>(raw, j);
+    sq += v * v;
+  }
+  sq += __shfl_xor(sq, 1, kWave);
+  sq += __shfl_xor(sq, 2, kWave);
+  // The conversion and the product each err by at most 2^-24.
+  if (in && wd % 4u == 0u)
+    norms[static_cast<size_t>(row) * (D / 32u) + wd / 4u] = static_cast<float>(sqrt(sq)) * (1.0f + 0x1p-22f) + 0x1p-140f;
+}
+
+// ---------------------------------------------------------------------------
 // Host-side launchers.
 
 int pow2_at_least(uint32_t v) {
@@ -1844,10 +2125,44 @@ int launch_route_rd(const osmd_moe_args& a, hipStream_t st) {
   return launch_status();
 }
 
+template <int RD, int NB>
+int launch_router_f64_range(const osmd_moe_args& a, const void* x, uint32_t x_bf16, const float* router_norms,
+                            const float* x_norms, float* planes, float* planes_lo, float* bound_planes,
+                            hipStream_t st) {
+  const uint32_t T = a.tokens, D = a.geom.hidden, E = a.expert_count;
+  const bool shared = (a.flags & OSMD_MOE_SHARED) != 0u;
+  const uint32_t gx = (E + (shared ? 1u : 0u) + 63u) / 64u, gz = D / (16u * NB);
+  const uint32_t gy = (T + 15u) / 16u;
+  const uint32_t launch = (gx * gy * gz + 7u) / 8u * 8u;
+  auto go = [&](auto kernel) {
+    kernel<<<launch, 256, 0, st>>>(x, T, D, a.router, shared ? a.shared_gate_vec : nullptr, E, a.router_group,
+                                   (a.flags & OSMD_MOE_RMSNORM) ? 1u : 0u, planes, planes_lo, router_norms, x_norms,
+                                   bound_planes, gx, gy, gz);
+  };
+  x_bf16 ? go(router_f64_kernel<RD, NB, true>) : go(router_f64_kernel<RD, NB, false>);
+  return launch_status();
+}
+
+template <int RD>
+int launch_router_f64(const osmd_moe_args& a, const void* x, uint32_t x_bf16, uint32_t cols, const float* router_norms,
+                      const float* x_norms, float* planes, float* planes_lo, float* bound_planes, hipStream_t st) {
+  if (cols == 0u || a.geom.hidden % cols != 0u) return static_cast<int>(hipErrorInvalidValue);
+  switch (cols) {
+    case 512:
+      return launch_router_f64_range<RD, 32>(a, x, x_bf16, router_norms, x_norms, planes, planes_lo, bound_planes, st);
+    case 256:
+      return launch_router_f64_range<RD, 16>(a, x, x_bf16, router_norms, x_norms, planes, planes_lo, bound_planes, st);
+    case 128:
+      return launch_router_f64_range<RD, 8>(a, x, x_bf16, router_norms, x_norms, planes, planes_lo, bound_planes, st);
+    default: return static_cast<int>(hipErrorInvalidValue);
+  }
+}
+
 RouteView route_view(const osmd_moe_args& a) {
   RouteView rv;
   rv.logits = a.logits;
   rv.planes = a.logit_planes;
+  rv.planes_lo = a.logit_planes_lo;
   rv.parts = a.logit_parts;
   rv.tokens = a.tokens;
   rv.logits_out = a.logits;
@@ -1930,6 +2245,39 @@ int osmd_moe_router(const osmd_moe_args* a, osmd_stream s) {
     case OSM_META_F16: return launch_route_rd<OSM_META_F16>(*a, st);
     case OSM_ROUTER_AFFINE_Q8: return launch_route_rd<OSM_ROUTER_AFFINE_Q8>(*a, st);
     default: return launch_route_rd<OSM_META_BF16>(*a, st);
+  }
+}
+
+int osmd_router_norms(const osmd_moe_args* a, float* norms, osmd_stream s) {
+  const uint32_t E = a->expert_count, D = a->geom.hidden;
+  const hipStream_t st = static_cast<hipStream_t>(s);
+  const dim3 grid((D / 8u + 255u) / 256u, E + ((a->flags & OSMD_MOE_SHARED) ? 1u : 0u));
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, 256, 0, st>>>(a->router, a->shared_gate_vec, E, D, a->router_group, norms);
+  };
+  switch (a->router_dtype) {
+    case OSM_META_F32: launch(router_norms_kernel<OSM_META_F32>); break;
+    case OSM_META_F16: launch(router_norms_kernel<OSM_META_F16>); break;
+    case OSM_ROUTER_AFFINE_Q8: launch(router_norms_kernel<OSM_ROUTER_AFFINE_Q8>); break;
+    default: return static_cast<int>(hipErrorInvalidValue);
+  }
+  return launch_status();
+}
+
+int osmd_router_f64(const osmd_moe_args* a, const void* x, uint32_t x_bf16, uint32_t parts, const float* router_norms,
+                    const float* x_norms, float* planes, float* planes_lo, float* bound_planes, osmd_stream s) {
+  const uint32_t cols = parts != 0u ? a->geom.hidden / parts : 0u;
+  switch (a->router_dtype) {
+    case OSM_META_F32:
+      return launch_router_f64<OSM_META_F32>(*a, x, x_bf16, cols, router_norms, x_norms, planes, planes_lo,
+                                             bound_planes, static_cast<hipStream_t>(s));
+    case OSM_META_F16:
+      return launch_router_f64<OSM_META_F16>(*a, x, x_bf16, cols, router_norms, x_norms, planes, planes_lo,
+                                             bound_planes, static_cast<hipStream_t>(s));
+    case OSM_ROUTER_AFFINE_Q8:
+      return launch_router_f64<OSM_ROUTER_AFFINE_Q8>(*a, x, x_bf16, cols, router_norms, x_norms, planes, planes_lo,
+                                                     bound_planes, static_cast<hipStream_t>(s));
+    default: return static_cast<int>(hipErrorInvalidValue);
   }
 }
 

@@ -1474,8 +1474,14 @@ int osmd_moe_grouped(const osmd_moe_grouped_args* a, osmd_stream s) {
   // GEMMs: 3 bf16 terms per activation for the router, of which the expert
   // GEMMs read the first 2 (the group sums are of those 2).
   const bool router_gemm = m.router_dtype == OSM_META_BF16 && (xbf16 || T > kRouterGemmMinTokens);
-  if (xbf16 && !router_gemm) {
-    // A router of another dtype runs as the per-token kernel, on fp32 input.
+  // A router of another dtype runs as a GEMM in fp64 from the automatic
+  // path's 40 tokens on, reading x itself (one 512-token pass of an 8-bit
+  // router: 400 µs as per-token GEMVs, 48 µs).
+  const bool router_f64 = m.router_dtype != OSM_META_BF16 && T >= OSMD_GROUPED_MIN_TOKENS &&
+                          a->logit_planes_lo != nullptr && a->router_norms != nullptr && a->x_norms != nullptr &&
+                          a->bound_planes != nullptr;
+  if (xbf16 && !router_gemm && !router_f64) {
+    // The per-token kernel takes fp32 input.
     const size_t n = static_cast<size_t>(T) * D;
     widen_bf16_kernel<<<blocks_for(n, 4096), 256, 0, st>>>(static_cast<const uint16_t*>(xin), n, m.x_norm);
     xin = m.x_norm;
@@ -1483,15 +1489,15 @@ int osmd_moe_grouped(const osmd_moe_grouped_args* a, osmd_stream s) {
   }
   // A bf16 input is exact as one bf16 term: the router GEMM and the gate/up
   // GEMM then read one term instead of three and two.
-  const bool one_term = router_gemm && xbf16;
-  const uint32_t x_term_count = router_gemm ? (one_term ? 1u : kRouterSplit) : kActSplit;
+  const bool one_term = (router_gemm || router_f64) && xbf16;
+  const uint32_t x_term_count = one_term ? 1u : router_gemm ? kRouterSplit : kActSplit;
   // Error bounds of the GEMM's logits need the router's and the input's
   // 32-column norms.
   const bool gemm_bounds = router_gemm && a->router_norms != nullptr && a->x_norms != nullptr &&
                            a->bound_planes != nullptr;
-  float* xnorms = gemm_bounds ? a->x_norms : nullptr;
+  float* xnorms = gemm_bounds || router_f64 ? a->x_norms : nullptr;
   const size_t words = static_cast<size_t>(T) * (D / 8u);
-  if (router_gemm) {
+  if (router_gemm || one_term) {
     if (one_term)
       prepare_kernel<true, 1><<<blocks_for(words, 4096), 256, 0, st>>>(xin, T, D, G, a->x_terms, a->x_sums, xnorms);
     else
@@ -1525,6 +1531,14 @@ int osmd_moe_grouped(const osmd_moe_grouped_args* a, osmd_stream s) {
     ms.logit_planes = a->logit_planes;
     ms.logit_parts = D / rcols;
     ms.bound_planes = gemm_bounds ? a->bound_planes : nullptr;
+  } else if (router_f64) {
+    ms.logit_parts = D / router_range(D);
+    r = osmd_router_f64(&m, xin, xbf16 ? 1u : 0u, ms.logit_parts, a->router_norms, xnorms, a->logit_planes,
+                        a->logit_planes_lo, a->bound_planes, s);
+    if (r != 0) return r;
+    ms.logit_planes = a->logit_planes;
+    ms.logit_planes_lo = a->logit_planes_lo;
+    ms.bound_planes = a->bound_planes;
   } else {
     // The decode router kernel, one token per grid row (fp32 input).
     osmd_moe_args ra = m;

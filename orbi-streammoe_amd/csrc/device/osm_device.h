@@ -155,6 +155,7 @@ typedef struct osmd_moe_args {
    * dot) that the selection adds in plane order, writing logits and
    * shared_gate itself; when null, logits and shared_gate are final. */
   const float* logit_planes;
+  const float* logit_planes_lo; /* what the planes' rounding to fp32 left, or null */
   uint32_t logit_parts;
   /* Routing exactness. logit_bounds [B, E]: the router writes, for every
    * logit, a bound on its distance from the reference's sequentially summed
@@ -260,7 +261,23 @@ typedef struct osmd_moe_grouped_args {
   const float* router_norms;
   float* x_norms;
   float* bound_planes;
+  /* Low parts of the logit planes of a router that is not bf16, the shape of
+   * logit_planes, or null: such a router then runs as one GEMV per token and
+   * row. */
+  float* logit_planes_lo;
 } osmd_moe_grouped_args;
+/* Tokens from which a layer's decodes take the grouped path by themselves,
+ * and from which a router that is not bf16 runs as a GEMM. */
+#define OSMD_GROUPED_MIN_TOKENS 40u
+/* Norms of a router's 32-column chunks, [E + 1][D/32] (row E only with a
+ * shared gate), each rounded up; any dtype but bf16. */
+int osmd_router_norms(const osmd_moe_args* a, float* norms, osmd_stream s);
+/* The router of a->tokens tokens as a GEMM in fp64, any dtype but bf16: x
+ * [T, D] (fp32, or bf16 when x_bf16; already normalised) against a->router
+ * and the shared gate, in `parts` = D / 512, 256 or 128 K ranges whose fp64
+ * sums go to planes + planes_lo, with the bound planes the selection reads. */
+int osmd_router_f64(const osmd_moe_args* a, const void* x, uint32_t x_bf16, uint32_t parts, const float* router_norms,
+                    const float* x_norms, float* planes, float* planes_lo, float* bound_planes, osmd_stream s);
 size_t osmd_moe_grouped_max_tiles(uint32_t tokens, uint32_t nslot, uint32_t experts);
 uint32_t osmd_moe_grouped_splits(const osm_expert_geometry* g, uint32_t cols);
 uint32_t osmd_moe_grouped_router_parts(uint32_t hidden);

@@ -122,7 +122,7 @@ struct HipMoeLayer::Impl {
   // workspace
   DeviceBytes x_in, y_out, logits, ids, weights, mass, shared_gate, x_norm, h, slot_ptrs;
   DeviceBytes logit_bounds;  // [T, E] bound of each logit's distance from the reference's
-  DeviceBytes router_norms;  // bf16 router: [E + 1][D/32] norms of its 32-column chunks (row E: shared gate)
+  DeviceBytes router_norms;  // [E + 1][D/32] norms of the router's 32-column chunks (row E: shared gate)
   DeviceBytes route_stats;   // 4 routing counters (osmd_moe_args::route_stats)
   PinnedBytes host_ptrs;  // staging for slot pointers chosen on the host
   PinnedBytes host_io;    // cache-driven path: pinned staging of inputs and outputs (grown on use)
@@ -154,7 +154,7 @@ struct HipMoeLayer::Impl {
   // workspace (every layer on one stream uses the same memory in turn)
   HipMoePath path = HipMoePath::automatic;
   enum GroupedBuf { kXTerms, kXSums, kPairPos, kPairW, kTiles, kTileCount, kGuPart, kHTerms, kHSums, kPartial,
-                    kLogitPlanes, kXNorms, kBoundPlanes, kGroupedBufs };
+                    kLogitPlanes, kXNorms, kBoundPlanes, kLogitPlanesLo, kGroupedBufs };
   std::array<std::size_t, kGroupedBufs> g_off{};
   std::size_t g_bytes = 0;
   std::uint8_t* g_base = nullptr;
@@ -175,7 +175,8 @@ struct HipMoeLayer::Impl {
         osmd_moe_grouped_splits(&g, static_cast<std::uint32_t>(I)) * P * D * 4U,   // down partials
         parts * T * (cfg.expert_count + 1U) * 4U,                                   // logit planes
         T * (D / 32U) * 4U,                                                         // input chunk norms
-        parts * T * (cfg.expert_count + 1U) * 4U};                                  // bound planes
+        parts * T * (cfg.expert_count + 1U) * 4U,                                   // bound planes
+        router_f64() ? parts * T * (cfg.expert_count + 1U) * 4U : 0U};              // low parts of the logit planes
     std::size_t off = 0;
     for (std::size_t i = 0; i < bytes.size(); ++i) {
       g_off[i] = off;
@@ -184,6 +185,11 @@ struct HipMoeLayer::Impl {
     g_bytes = off;
   }
 
+  // Layers whose router is not bf16 and that can take batches of the router
+  // GEMM's size run it in fp64.
+  bool router_f64() const {
+    return router_dtype != OSM_META_BF16 && max_tokens >= kGroupedMinTokens && grouped_ok(nullptr);
+  }
   int ensure_grouped(HipComputeContext& context) {
     if (g_bytes == 0) plan_grouped();
     int rc = 0;
@@ -223,6 +229,7 @@ struct HipMoeLayer::Impl {
     ga.router_norms = router_norms.as<const float>();
     ga.x_norms = gbuf<float>(kXNorms);
     ga.bound_planes = gbuf<float>(kBoundPlanes);
+    ga.logit_planes_lo = router_f64() ? gbuf<float>(kLogitPlanesLo) : nullptr;
     return ga;
   }
 
@@ -418,6 +425,11 @@ std::optional<HipMoeLayer> HipMoeLayer::create(HipComputeContext& context, const
     if (rc == 0) rc = osmd_zero(impl->slot_ptrs.get(), impl->slot_ptrs.size(), st);
     if (rc == 0) rc = osmd_zero(impl->shared_gate.get(), T * sizeof(float), st);
     if (rc == 0) rc = impl->host_ptrs.allocate(T * nslot * sizeof(void*));
+    if (rc == 0 && impl->router_f64()) {
+      rc = impl->router_norms.allocate((E + 1U) * (D / 32U) * sizeof(float));
+      const osmd_moe_args a = impl->args(nullptr, nullptr, 0U, nullptr, false);
+      if (rc == 0) rc = osmd_router_norms(&a, impl->router_norms.as<float>(), st);
+    }
     if (rc == 0) rc = osmd_stream_synchronize(st);
     if (rc != 0) {
       set_diag(diagnostic, hip_error("MoE layer allocation/upload failed", rc));

@@ -792,7 +792,7 @@ struct HipMoeResult {
 // 40: 201-207 vs 198; 48: 213-218 vs 211; 64: 266-272 vs 239; 512: 2730 vs
 // 387).
 enum class HipMoePath { automatic = 0, per_token = 1, grouped = 2 };
-inline constexpr std::uint32_t kGroupedMinTokens = 40;
+inline constexpr std::uint32_t kGroupedMinTokens = OSMD_GROUPED_MIN_TOKENS;
 
 class HipMoeLayer {
  public:

@@ -1,0 +1,72 @@
+"""Routers that are not bf16 through the fp64 router GEMM: every token's
+picks against the oracle's, at the K ranges, token tiles and router rows
+where the GEMM's edges lie."""
+
+import numpy as np
+import pytest
+
+import oracle as O
+import osm_hip
+from helpers import max_abs
+from test_gpu_router_q8 import dequant, quantize_q8
+
+pytestmark = pytest.mark.gpu
+
+
+def layer(ctx, kind, D, E, k, T, seed):
+    rng = np.random.default_rng(seed)
+    I, G = 128, 64
+    g = osm_hip.geometry(D, I, G, osm_hip.BF16)
+    slab = osm_hip.ExpertSlab(ctx, g, 1, E)
+    slab.synthesize(seed)
+    shared = O.synth_expert_blob(seed, 0, O.SHARED_EXPERT_ID, D, I, G)
+    w = rng.normal(0, 0.9 / np.sqrt(D), (E + 1, D)).astype(np.float32)
+    w[1] = w[0] * np.float32(1 + 2.0**-21)  # a pair whose logits the bounds cannot tell apart
+    if kind == "q8":
+        r, sg = quantize_q8(w[:-1], 64, rng), quantize_q8(w[-1:], 64, rng)
+        value, gate = dequant(*r, 64), dequant(*sg, 64)
+        moe = osm_hip.MoeLayer(ctx, g, E, k, r + (64,), osm_hip.AFFINE_Q8, sg + (64,), None, shared, max_tokens=T)
+    else:
+        dt, code = (np.float16, osm_hip.F16) if kind == "f16" else (np.float32, osm_hip.F32)
+        w = w.astype(dt)
+        value, gate = w[:-1].astype(np.float32), w[-1:].astype(np.float32)
+        moe = osm_hip.MoeLayer(ctx, g, E, k, w[:-1], code, w[-1], None, shared, max_tokens=T)
+    return slab, moe, value, gate
+
+
+def check(moe, x, value, gate, E, k):
+    r = moe.routing(len(x))
+    exact = x.astype(np.float64) @ value.astype(np.float64).T
+    # Summed in fp64 and rounded to fp32 once, whatever of the planes' 48 bits is lost below that.
+    bound = 2.0**-24 * np.abs(exact) + 2.0**-40 * (np.abs(x).astype(np.float64) @ np.abs(value).astype(np.float64).T)
+    assert np.all(np.abs(r["logits"] - exact) <= bound)
+    for t in range(len(x)):
+        ora = O.route_qwen_top_k(x[t], value, x.shape[1], E, k, True)
+        assert np.array_equal(r["ids"][t], ora["ids"]), t
+        # The weights are the picks' softmax of the logits checked above, each exp, sum and quotient rounded.
+        p = np.exp(r["logits"][t][ora["ids"]].astype(np.float64) - r["logits"][t].max())
+        assert max_abs(r["weights"][t], p / p.sum()) <= 1e-6
+    s = 1 / (1 + np.exp(-(x.astype(np.float64) @ gate[0].astype(np.float64))))
+    assert max_abs(r["shared_gate"], s) <= 2e-6
+
+
+# D 2048, 768 and 384: K ranges of 512, 256 and 128 columns. E + 1 rows fill a 64-row block, or leave one row in the
+# next. 40 tokens are the fewest, 49 leave
+# one in the fourth tile, 257 take two tiles per workgroup and leave one.
+@pytest.mark.parametrize("D,E,T", [(2048, 128, 49), (768, 63, 40), (384, 64, 257), (2048, 512, 64)])
+@pytest.mark.parametrize("kind", ["q8", "f32", "f16"])
+def test_router_f64(ctx, D, E, T, kind):
+    k, seed = 6, 900 + D + T
+    slab, moe, value, gate = layer(ctx, kind, D, E, k, T, seed)
+    x = O.synth_tokens(seed, 0, T, D)
+    xd, yd = ctx.alloc(T * D * 4), ctx.alloc(T * D * 4)
+    xd.upload(x)
+    moe.set_path(osm_hip.PATH_GROUPED)
+    moe.routing_stats(reset=True)
+    moe.decode_device(slab, 0, xd.ptr, yd.ptr, T)
+    check(moe, x, value, gate, E, k)
+    assert moe.routing_stats()["exact"] < T  # the bounds prove some of them
+    bits = ((x.view(np.uint32) + 0x7FFF + ((x.view(np.uint32) >> 16) & 1)) >> 16).astype(np.uint16)
+    xd.upload(bits)
+    moe.prefill_device(slab, 0, xd.ptr, yd.ptr, T)
+    check(moe, (bits.astype(np.uint32) << 16).view(np.float32).reshape(T, D), value, gate, E, k)
