@@ -437,7 +437,7 @@ __device__ float exact_rms_scale(const RouteView& rv, uint32_t t, Selection<PER>
     __syncthreads();
   }
   if (threadIdx.x == 0)
-    out.scal[1] = __fdiv_rn(1.0f, __fsqrt_rn(__fdiv_rn(ss, static_cast<float>(rv.hidden)) + rv.rms_eps));
+    out.scal[1] = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(ss, static_cast<float>(rv.hidden)) + rv.rms_eps));
   __syncthreads();
   return out.scal[1];
 }
