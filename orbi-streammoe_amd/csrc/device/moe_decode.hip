@@ -290,6 +290,18 @@ constexpr uint32_t kExactSegs = (kSelThreads - kWave) / kExactRows;  // producer
 constexpr uint32_t kExactCols = kExactSegs * 16u;                     // 192 columns per chunk
 constexpr uint32_t kExactStride = kExactCols + 4u;  // LDS row stride: 16-byte aligned rows, adders' reads in distinct banks
 
+// A chain split over the workgroup (chain_split): chunks of the chain, one to
+// each half wavefront, and the start values tried for each, one to a lane.
+constexpr uint32_t kSplitChunks = 2u * kSelWaves;
+constexpr uint32_t kSplitTries = 32;
+// Its products are two rows of up to this many columns in the exact path's
+// product buffer, the chunks' results behind them.
+constexpr uint32_t kSplitMaxCols = 2048;
+static_assert((2u * kSplitMaxCols + 2u * kSplitChunks * kSplitTries) <= 2u * kExactRows * kExactStride,
+              "the split chain's rows and results fit the product buffer");
+static_assert(kSplitMaxCols <= 8u * kSelThreads, "one word of 8 columns per thread");
+constexpr uint32_t kMaxOpen = 6;  // experts whose order resolve_clusters settles
+
 // Bins of the device ranking's distance histogram (rank_device).
 constexpr uint32_t kHistBins = 64;
 constexpr float kHistSpan = 256.0f;
@@ -318,6 +330,13 @@ struct Selection {
   uint32_t nneartie, ncand, thr, flags, wcount[kSelWaves];  // nneartie: near ties sent to the full recompute
   uint32_t again;                             // exact path: recompute every expert
   uint16_t cl[kSelThreads * PER];             // exact path: candidate list
+  // Exact path on the open clusters alone (resolve_clusters): their members,
+  // the reference's logit of each, each one's first rank in its cluster, and
+  // chain_split's chunk sums and centres.
+  uint32_t uid[kMaxOpen], ustart[kMaxOpen], nopen;
+  float uval[kMaxOpen];
+  double csum[2][kSplitChunks];
+  uint32_t ccen[2][kSplitChunks];
   __attribute__((aligned(16))) float xe[2][kExactCols];  // exact path: the inputs of two chunks
   __attribute__((aligned(16))) float prod[2][kExactRows][kExactStride];  // exact path: rounded products of two chunks
 };
@@ -415,6 +434,264 @@ __device__ __forceinline__ float x1_value(const RouteView& rv, uint32_t bits) {
   return rv.x_bf16 ? bf16_to_f32(bits) : __uint_as_float(bits);
 }
 
+// Place of column c in a row of chain_split: the 4 x 4 transpose of each run
+// of 16, so that lane l % 4 of a quad reads columns l, 4 + l, 8 + l, 12 + l of
+// the run together.
+__device__ __forceinline__ uint32_t split_place(uint32_t c) {
+  return (c & ~15u) | ((c & 3u) << 2) | ((c >> 2) & 3u);
+}
+// a + the four lanes' values of x in lane order, and b likewise of y: quad
+// broadcasts as DPP operands of the additions.
+template <int CTRL>
+__device__ __forceinline__ float quad_value(float v) {  // every lane has a source: one v_add_f32 with a DPP operand
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ void add4(float x, float& a, float y, float& b) {
+#pragma clang fp contract(off)
+  a = a + quad_value<0x00>(x);
+  b = b + quad_value<0x00>(y);
+  a = a + quad_value<0x55>(x);
+  b = b + quad_value<0x55>(y);
+  a = a + quad_value<0xAA>(x);
+  b = b + quad_value<0xAA>(y);
+  a = a + quad_value<0xFF>(x);
+  b = b + quad_value<0xFF>(y);
+}
+
+// Sums of two rows of n fp32 values (LDS, row m at prod + m n, 16-byte
+// aligned, columns at split_place; n a multiple of 128, at most
+// kSplitMaxCols) exactly as one chain adds them: from +0 in order, each
+// addition rounded. Every thread of the workgroup
+// calls it; result[0] and result[1] in LDS are complete when it returns.
+//
+// One chain of 2,048 dependent additions takes 9 µs, and the launch waits for
+// its slowest token. Here eight chunks of it run side by side. A chunk's start, the rounded sum of the chunks before,
+// is not known, but it is near their exact sum: the 32 lanes of a half
+// wavefront run the chunk from the 32 fp32 values around it. Then the chunks
+// are put together in order: the running value is looked up among a chunk's
+// start values, bit for bit, and replaced by what that lane's chain came to.
+// Where it is none of them (after a partial sum close to zero, whose
+// neighbours lie closer together than the rounding before it) the chunk is
+// run once more from the running value itself. Either way every addition of
+// the result was made from the value the chain has there.
+//
+// A pass over two rows takes 3 to 4 µs. Few launches run this code twice on a
+// compute unit, so fetching it counts as much as running it: loops stay
+// rolled and there is one copy (with the look-ups' second runs unrolled a pair
+// took 4 µs more). Selection launches, one chain / this, kernel trace: 64
+// tokens with RMSNorm 35 / 29 µs, 512 with an 8-bit router 46 / 34; without the
+// norm (512 bf16 tokens) 28 / 28.
+template <int PER>
+__device__ __forceinline__ void chain_split(const float* prod, uint32_t n, float* tab, Selection<PER>& out,
+                                            float* result) {
+#pragma clang fp contract(off)
+  const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const uint32_t hl = lane % kSplitTries, chunk = tid / kSplitTries;
+  const uint32_t len4 = n / (4u * kSplitChunks);
+  const float4* r0 = reinterpret_cast<const float4*>(prod) + chunk * len4;
+  const float4* r1 = r0 + n / 4u;
+  double s0 = 0.0, s1 = 0.0;
+#pragma unroll 1
+  for (uint32_t i = hl; i < len4; i += kSplitTries) {
+    const float4 a = r0[i], b = r1[i];
+    s0 += (static_cast<double>(a.x) + a.y) + (static_cast<double>(a.z) + a.w);
+    s1 += (static_cast<double>(b.x) + b.y) + (static_cast<double>(b.z) + b.w);
+  }
+  s0 += dpp_d<kDppXor1>(s0);
+  s1 += dpp_d<kDppXor1>(s1);
+  s0 += dpp_d<kDppXor2>(s0);
+  s1 += dpp_d<kDppXor2>(s1);
+  s0 += dpp_d<kDppRowHalfMirror>(s0);
+  s1 += dpp_d<kDppRowHalfMirror>(s1);
+  s0 += dpp_d<kDppRowMirror>(s0);
+  s1 += dpp_d<kDppRowMirror>(s1);
+  s0 += dpp_d<kDppRowBcast15, 0xA>(s0);  // lanes 16-31 and 48-63: the half wavefront's
+  s1 += dpp_d<kDppRowBcast15, 0xA>(s1);
+  if (hl == kSplitTries - 1u) {
+    out.csum[0][chunk] = s0;
+    out.csum[1][chunk] = s1;
+  }
+  __syncthreads();
+  // The chunks before this one, summed over each eight lanes.
+  static_assert(kSplitChunks == 8u, "eight lanes hold the chunks' sums");
+  s0 = hl % 8u < chunk ? out.csum[0][hl % 8u] : 0.0;
+  s1 = hl % 8u < chunk ? out.csum[1][hl % 8u] : 0.0;
+  s0 += dpp_d<kDppXor1>(s0);
+  s1 += dpp_d<kDppXor1>(s1);
+  s0 += dpp_d<kDppXor2>(s0);
+  s1 += dpp_d<kDppXor2>(s1);
+  s0 += dpp_d<kDppRowHalfMirror>(s0);
+  s1 += dpp_d<kDppRowHalfMirror>(s1);
+  const uint32_t c0 = __float_as_uint(static_cast<float>(s0)), c1 = __float_as_uint(static_cast<float>(s1));
+  if (hl == 0u) {
+    out.ccen[0][chunk] = c0;
+    out.ccen[1][chunk] = c1;
+  }
+  float a0 = chunk == 0u ? 0.0f : __uint_as_float(c0 + hl - kSplitTries / 2u);
+  float a1 = chunk == 0u ? 0.0f : __uint_as_float(c1 + hl - kSplitTries / 2u);
+  // A lane reads a quarter of the chunk, 16 columns' in one load, and takes
+  // the rest from its quad's other lanes as DPP operands, a quarter of the LDS
+  // reads.
+  const uint32_t ql = lane % 4u;
+  float4 p0 = r0[ql], p1 = r1[ql];
+#pragma unroll 1
+  for (uint32_t i = 4u; i <= len4; i += 4u) {
+    const float4 q0 = p0, q1 = p1;
+    const uint32_t k = i < len4 ? i + ql : ql;  // the last round reads the first again
+    p0 = r0[k];
+    p1 = r1[k];
+    __builtin_amdgcn_sched_barrier(0);
+    add4(q0.x, a0, q1.x, a1);
+    add4(q0.y, a0, q1.y, a1);
+    add4(q0.z, a0, q1.z, a1);
+    add4(q0.w, a0, q1.w, a1);
+  }
+  tab[chunk * kSplitTries + hl] = a0;
+  tab[(kSplitChunks + chunk) * kSplitTries + hl] = a1;
+  __syncthreads();
+  if (wave < 2u) {  // wavefront m puts row m together; the running value is uniform
+    const float* ends = tab + wave * kSplitChunks * kSplitTries + hl;
+    float v = readlane_f(ends[0], 0);
+    float next = ends[kSplitTries];
+    uint32_t centre = out.ccen[wave][1];
+#pragma unroll 1
+    for (uint32_t c = 1; c < kSplitChunks; ++c) {
+      const float end = next;
+      const uint32_t idx = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+          static_cast<int>(__float_as_uint(v) - centre + kSplitTries / 2u)));
+      const uint32_t cn = c + 1u < kSplitChunks ? c + 1u : c;
+      next = ends[cn * kSplitTries];
+      centre = out.ccen[wave][cn];
+      if (idx < kSplitTries) {
+        v = readlane_f(end, static_cast<int>(idx));
+      } else {
+        const float4* r = reinterpret_cast<const float4*>(prod + wave * n) + c * len4;
+        float none = 0.0f;
+#pragma unroll 1
+        for (uint32_t i = 0; i < len4; i += 4u) {
+          const float4 p = r[i + ql];
+          add4(p.x, v, 0.0f, none);
+          add4(p.y, v, 0.0f, none);
+          add4(p.z, v, 0.0f, none);
+          add4(p.w, v, 0.0f, none);
+        }
+      }
+    }
+    if (lane == 0) result[wave] = v;
+  }
+  __syncthreads();
+}
+
+// 8 router elements of row e at column c as loaded, and their values, for any
+// router dtype.
+struct RowWord {
+  uint4 a, b;  // affine q8: two words, then their scales; their biases
+};
+__device__ __forceinline__ RowWord load_row_word(const RouteView& rv, uint32_t e, uint32_t c) {
+  RowWord r;
+  if (rv.router_dtype == OSM_ROUTER_AFFINE_Q8) {
+    Raw8<OSM_ROUTER_AFFINE_Q8> w;
+    load_q8x8(q8_row(rv.router, rv.expert_count, e, rv.hidden, rv.router_group), c, w);
+    r.a = make_uint4(w.q.x, w.q.y, __float_as_uint(w.s[0]), __float_as_uint(w.s[1]));
+    r.b = make_uint4(__float_as_uint(w.b[0]), __float_as_uint(w.b[1]), 0u, 0u);
+  } else {
+    const bool f32 = rv.router_dtype == OSM_META_F32;
+    const uint8_t* p = static_cast<const uint8_t*>(rv.router) +
+                       (static_cast<size_t>(e) * rv.hidden + c) * (f32 ? 4u : 2u);
+    r.a = ldg16(p);
+    r.b = ldg16(f32 ? p + 16 : p);
+  }
+  return r;
+}
+__device__ __forceinline__ void row_word_values(const RouteView& rv, const RowWord& r, float (&w)[8]) {
+  const uint32_t v[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+  const uint32_t dt = rv.router_dtype;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t half = (v[j / 2] >> (16 * (j % 2))) & 0xFFFFu;
+    if (dt == OSM_META_F32)
+      w[j] = __uint_as_float(v[j]);
+    else if (dt == OSM_META_F16)
+      w[j] = f16_to_f32(half);
+    else if (dt == OSM_ROUTER_AFFINE_Q8)
+      w[j] = dequant_q8(__uint_as_float(v[2 + j / 4]), static_cast<float>((v[j / 4] >> (8 * (j % 4))) & 0xFFu),
+                        __uint_as_float(v[4 + j / 4]));
+    else
+      w[j] = bf16_to_f32(half);
+  }
+}
+
+// The reference's logits of out.uid[0 .. n) (1 <= n <= kMaxOpen) for token t, rows
+// of up to kSplitMaxCols columns, two at a time in out.uval; in the sublayer
+// form the RMS scale's sum of squares is the first pass. A thread takes 8
+// columns (threads past the row read column 0's and write nothing).
+template <int PER>
+__device__ __forceinline__ void split_logits(const RouteView& rv, uint32_t t, Selection<PER>& out, uint32_t n) {
+#pragma clang fp contract(off)
+  static_assert(kSplitMaxCols <= 8u * kSelThreads, "8 columns per thread");
+  const uint32_t D = rv.hidden;
+  const bool in_row = 8u * threadIdx.x < D;
+  const uint32_t c = in_row ? 8u * threadIdx.x : 0u;
+  float* prod = &out.prod[0][0][0];
+  float x[8];
+  const size_t o = static_cast<size_t>(t) * D + c;
+  if (rv.x_bf16) {
+    const uint4 h = ldg16(reinterpret_cast<const uint16_t*>(rv.x) + o);
+    const uint32_t w[4] = {h.x, h.y, h.z, h.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = bf16_to_f32((w[j / 2] >> (16 * (j % 2))) & 0xFFFFu);
+  } else {
+    const uint4 f = ldg16(reinterpret_cast<const float*>(rv.x) + o), g = ldg16(reinterpret_cast<const float*>(rv.x) + o + 4u);
+    const uint32_t w[8] = {f.x, f.y, f.z, f.w, g.x, g.y, g.z, g.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = __uint_as_float(w[j]);
+  }
+  uint4 n0 = make_uint4(0u, 0u, 0u, 0u), n1 = n0;
+  if (rv.rms) {
+    n0 = ldg16(rv.norm_weight + c);
+    n1 = ldg16(rv.norm_weight + c + 4u);
+  }
+  RowWord wa = load_row_word(rv, out.uid[0], c), wb = load_row_word(rv, out.uid[n > 1u ? 1u : 0u], c);
+  uint32_t i0 = 0u;
+  bool squares = rv.rms != 0u;
+#pragma unroll 1
+  while (i0 < n) {
+    float a[8], b[8];
+    if (squares) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[j] = b[j] = x[j];
+    } else {
+      row_word_values(rv, wa, a);
+      row_word_values(rv, wb, b);
+      if (i0 + 2u < n) {
+        wa = load_row_word(rv, out.uid[i0 + 2u], c);
+        wb = load_row_word(rv, out.uid[i0 + 3u < n ? i0 + 3u : i0 + 2u], c);
+      }
+    }
+    if (in_row) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t at = split_place(c) + split_place(j);  // c is a multiple of 8
+        prod[at] = a[j] * x[j];
+        prod[D + at] = b[j] * x[j];
+      }
+    }
+    __syncthreads();
+    chain_split(prod, D, prod + 2u * kSplitMaxCols, out, out.uval + i0);
+    if (squares) {
+      // The scale and the scaled input, each operation rounded as the
+      // reference's (reference_ops.cpp:113-126).
+      squares = false;
+      const float scale = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(out.uval[0], static_cast<float>(D)) + rv.rms_eps));
+      const uint32_t w[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = x[j] * (scale * __uint_as_float(w[j]));
+    } else {
+      i0 += 2u;
+    }
+  }
+}
+
 // The reference's RMSNorm scale of token t: the squares summed in order,
 // then 1 / sqrt(sum / D + eps), each operation rounded to fp32
 // (reference_ops.cpp:113-121). Every thread calls it; x is staged in LDS
@@ -504,8 +781,9 @@ __device__ void exact_logits_rd(const RouteView& rv, uint32_t t, Selection<PER>&
   fetch_x(kExactCols);
   __syncthreads();
   float acc = 0.0f;
-  // The adders' wavefront issues first on its SIMD while it adds (as in
-  // exact_logits_deep).
+  // The adders' wavefront issues first on its SIMD while it adds: each
+  // addition waits for the one before it, and a wavefront of another
+  // workgroup sharing the SIMD would otherwise take the slots in between.
   const bool adder_wave = tid < kWave;
   if (adder_wave) __builtin_amdgcn_s_setprio(2);
   for (uint32_t k = 0; k <= nchunks; ++k) {
@@ -536,136 +814,121 @@ __device__ void exact_logits_rd(const RouteView& rv, uint32_t t, Selection<PER>&
   if (tid < nr) out.ex[out.cl[first + tid]] = acc;
 }
 
-// The same logits with the loads two steps ahead: router elements in two
-// register sets used on alternate steps, inputs loaded two steps before they
-// are staged, and additions in batches of 64. For the selection kernel (one
-// workgroup per token, registers to spare): a step is then the addition chain
-// rather than the producers' wait for their loads.
-template <int RD, int PER>
-__device__ void exact_logits_deep(const RouteView& rv, uint32_t t, Selection<PER>& out, uint32_t first, uint32_t nr,
-                                  float scale) {
-#pragma clang fp contract(off)
-  const uint32_t D = rv.hidden, tid = threadIdx.x;
-  const bool producer = tid >= kWave;
-  const uint32_t ptid = producer ? tid - kWave : 0u;
-  const uint32_t r = ptid % kExactRows, seg = (ptid / kExactRows) * 16u;
-  const bool active = producer && r < nr;
-  const uint32_t e = r < nr ? out.cl[first + r] : out.cl[first];
-  Q8Row qr{};
-  const uint8_t* row = nullptr;
-  if constexpr (RD == OSM_ROUTER_AFFINE_Q8)
-    qr = q8_row(rv.router, rv.expert_count, e, D, rv.router_group);
-  else
-    row = static_cast<const uint8_t*>(rv.router) + static_cast<size_t>(e) * D * (RD == OSM_META_F32 ? 4u : 2u);
-  struct W16 {
-    Raw8<RD> lo, hi;
-  };
-  struct X1 {
-    uint32_t x;  // as loaded (load_x1_bits)
-    float nw;
-  };
-  auto fetch_w = [&](W16& w, uint32_t chunk) {
-    const uint32_t c = chunk * kExactCols + seg;
-    if (!active) return;
-    if (c < D) {
-      if constexpr (RD == OSM_ROUTER_AFFINE_Q8) load_q8x8(qr, c, w.lo); else load_raw8<RD>(row, c, w.lo);
-    }
-    if (c + 8u < D) {
-      if constexpr (RD == OSM_ROUTER_AFFINE_Q8) load_q8x8(qr, c + 8u, w.hi); else load_raw8<RD>(row, c + 8u, w.hi);
-    }
-  };
-  auto fetch_x = [&](X1& v, uint32_t chunk) {
-    if (!producer) return;
-    const uint32_t c = chunk * kExactCols + ptid;
-    v.x = load_x1_bits(rv, t, c);
-    v.nw = (rv.rms && c < D) ? ldg<float>(rv.norm_weight + c) : 1.0f;
-  };
-  auto stage_x = [&](const X1& v, uint32_t buf) {
-    if (!producer) return;
-    const float xv = x1_value(rv, v.x);
-    out.xe[buf][ptid] = rv.rms ? xv * (scale * v.nw) : xv;
-  };
-  const uint32_t nchunks = (D + kExactCols - 1u) / kExactCols;
-  float acc = 0.0f;
-  // Step k: products of chunk k from w (loaded in step k - 2), w refilled
-  // with chunk k + 2; chunk k + 1's inputs staged from xs (loaded in step
-  // k - 2), xs refilled with chunk k + 3; lane r of wavefront 0 adds chunk
-  // k - 1.
-  auto step = [&](uint32_t k, W16& w, X1& xs) {
-    if (active && k < nchunks) {
-      float4* dst = reinterpret_cast<float4*>(&out.prod[k & 1u][r][seg]);
-      const float4* xe = reinterpret_cast<const float4*>(&out.xe[k & 1u][seg]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float4 x4 = xe[j];
-        const Raw8<RD>& h = j < 2 ? w.lo : w.hi;
-        const int o = 4 * (j % 2);
-        dst[j] = make_float4(raw8_get<RD>(h, o) * x4.x, raw8_get<RD>(h, o + 1) * x4.y,
-                             raw8_get<RD>(h, o + 2) * x4.z, raw8_get<RD>(h, o + 3) * x4.w);
-      }
-      if (k + 2u < nchunks) fetch_w(w, k + 2u);
-    }
-    if (k + 1u < nchunks) {
-      stage_x(xs, (k + 1u) & 1u);
-      if (k + 3u < nchunks) fetch_x(xs, k + 3u);
-    }
-    if (tid < nr && k > 0u) {
-      const uint32_t c0 = (k - 1u) * kExactCols;
-      acc = chain_sum<16>(out.prod[(k - 1u) & 1u][tid], D - c0 < kExactCols ? D - c0 : kExactCols, acc);
-    }
-    __syncthreads();
-  };
-  W16 wa{}, wb{};
-  X1 xa{}, xb{};
-  fetch_x(xa, 0);
-  fetch_w(wa, 0);
-  if (nchunks > 1u) fetch_w(wb, 1);
-  stage_x(xa, 0);
-  if (nchunks > 1u) fetch_x(xb, 1);
-  if (nchunks > 2u) fetch_x(xa, 2);
-  __syncthreads();
-  // The adders' wavefront issues first on its SIMD while it adds: each
-  // addition waits for the one before it, and a wavefront of another
-  // workgroup sharing the SIMD would otherwise take the slots in between.
-  const bool adder_wave = tid < kWave;
-  if (adder_wave) __builtin_amdgcn_s_setprio(2);
-  // Even steps stage odd chunks from xb, odd steps even chunks from xa.
-  for (uint32_t k = 0; k <= nchunks; k += 2u) {
-    step(k, wa, xb);
-    if (k + 1u <= nchunks) step(k + 1u, wb, xa);
-  }
-  if (adder_wave) __builtin_amdgcn_s_setprio(0);
-  if (tid < nr) out.ex[out.cl[first + tid]] = acc;
-}
-
-template <int PER, bool DEEP>
+template <int PER>
 __device__ void exact_logits(const RouteView& rv, uint32_t t, Selection<PER>& out, uint32_t first, uint32_t nr,
                              float scale) {
   switch (rv.router_dtype) {
-    case OSM_META_F32:
-      if constexpr (DEEP) exact_logits_deep<OSM_META_F32>(rv, t, out, first, nr, scale);
-      else exact_logits_rd<OSM_META_F32>(rv, t, out, first, nr, scale);
-      break;
-    case OSM_META_F16:
-      if constexpr (DEEP) exact_logits_deep<OSM_META_F16>(rv, t, out, first, nr, scale);
-      else exact_logits_rd<OSM_META_F16>(rv, t, out, first, nr, scale);
-      break;
-    case OSM_ROUTER_AFFINE_Q8:
-      if constexpr (DEEP) exact_logits_deep<OSM_ROUTER_AFFINE_Q8>(rv, t, out, first, nr, scale);
-      else exact_logits_rd<OSM_ROUTER_AFFINE_Q8>(rv, t, out, first, nr, scale);
-      break;
-    default:
-      if constexpr (DEEP) exact_logits_deep<OSM_META_BF16>(rv, t, out, first, nr, scale);
-      else exact_logits_rd<OSM_META_BF16>(rv, t, out, first, nr, scale);
-      break;
+    case OSM_META_F32: exact_logits_rd<OSM_META_F32>(rv, t, out, first, nr, scale); break;
+    case OSM_META_F16: exact_logits_rd<OSM_META_F16>(rv, t, out, first, nr, scale); break;
+    case OSM_ROUTER_AFFINE_Q8: exact_logits_rd<OSM_ROUTER_AFFINE_Q8>(rv, t, out, first, nr, scale); break;
+    default: exact_logits_rd<OSM_META_BF16>(rv, t, out, first, nr, scale); break;
   }
+}
+
+// The exact path for rankings that the bounds leave open in a few places (a
+// near tie or two: nearly all of them). The candidates (out.cl, nc of them) are
+// ordered by device logit; a cut lies after rank r where the lowest lower bound
+// of ranks 0 .. r is above the highest upper bound, with the tie margin, of all
+// ranks after it. What a cut separates the reference orders alike, whatever
+// the order within. Between cuts lie clusters: one of a single expert is in
+// its place; the reference's logits of the others, if they are at most
+// kMaxOpen and reach the first k ranks, are summed as it sums them, and order
+// their cluster: by the logit, equal ones by id. Two neighbours of different
+// logit whose lower one has the lower id must be apart by the tie margin, or
+// their probabilities might be equal. True when out.id and out.lg are then the
+// reference's; false (nothing written) where the general form below is needed.
+// Every thread of the workgroup calls it.
+template <int PER>
+__device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>& out, float mx, uint32_t nc) {
+  const uint32_t k = rv.top_k, tid = threadIdx.x, lane = tid % kWave;
+  uint32_t e = 0u, start = 0u, upos = 0u;
+  bool open = false;
+  if (tid < kWave) {
+    // Lane i: candidate i of the list, then the candidate of rank i.
+    const uint32_t e0 = lane < nc ? out.cl[lane] : 0u;
+    const float l0 = lane < nc ? out.val[e0] : -INFINITY;
+    bool fine = lane >= nc || (l0 - l0 == 0.0f && out.aux[e0] < INFINITY);
+    uint32_t rk = 0u;
+#pragma unroll 1
+    for (uint32_t i = 0; i < nc; ++i) {
+      const float li = readlane_f(l0, static_cast<int>(i));
+      const uint32_t ei = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(e0), static_cast<int>(i)));
+      rk += (li > l0 || (li == l0 && ei < e0)) ? 1u : 0u;
+    }
+    fine = __all(fine) != 0;
+    if (fine && lane < nc) out.cand[rk] = e0;  // the ranking's keys are done with
+    __builtin_amdgcn_wave_barrier();
+    float l = -INFINITY, b = 0.0f;
+    if (fine && lane < nc) {
+      e = static_cast<uint32_t>(out.cand[lane]);
+      l = out.val[e];
+      b = out.aux[e];
+    }
+    const float lo = l - kBoundSlack * b, hi = l + kBoundSlack * b + tie_margin(mx, l);
+    float low = INFINITY, high = -INFINITY;
+#pragma unroll 1
+    for (uint32_t i = 0; i < nc; ++i) {
+      const float li = readlane_f(lo, static_cast<int>(i)), hj = readlane_f(hi, static_cast<int>(i));
+      low = i <= lane ? fminf(low, li) : low;
+      high = i > lane ? fmaxf(high, hj) : high;
+    }
+    const uint64_t cuts = __ballot(lane < nc && low > high);
+    const uint64_t below = cuts & ((1ull << lane) - 1ull);
+    start = below ? 64u - static_cast<uint32_t>(__builtin_clzll(below)) : 0u;
+    open = lane < nc && start < k && !(start == lane && ((cuts >> lane) & 1ull));
+    const uint64_t all = __ballot(open);
+    upos = static_cast<uint32_t>(__popcll(all & ((1ull << lane) - 1ull)));
+    const uint32_t n = static_cast<uint32_t>(__popcll(all));
+    if (lane == 0) out.nopen = fine && n <= kMaxOpen ? n : ~0u;
+    if (open && upos < kMaxOpen) {
+      out.uid[upos] = e;
+      out.ustart[upos] = start;
+    }
+  }
+  __syncthreads();
+  const uint32_t n = out.nopen;
+  if (n == ~0u) return false;
+  if (n > 0u) split_logits(rv, t, out, n);
+  if (tid < kWave) {
+    uint32_t rank = lane;
+    bool bad = false;
+    if (open) {
+      const float v = out.uval[upos];
+      rank = start;
+      float nv = -INFINITY;  // the next lower of the cluster
+      uint32_t ne = 0u;
+#pragma unroll 1
+      for (uint32_t i = 0; i < n; ++i) {
+        if (out.ustart[i] != start || i == upos) continue;
+        const float w = out.uval[i];
+        const uint32_t ei = out.uid[i];
+        const bool above = w > v || (w == v && ei < e);
+        if (above) {
+          ++rank;
+        } else if (w > nv || (w == nv && ei < ne)) {
+          nv = w;
+          ne = ei;
+        }
+      }
+      bad = !(v - v == 0.0f) ||
+            (rank < k && nv > -INFINITY && v != nv && e > ne && !(v - nv > tie_margin(mx, nv)));
+    }
+    bad = __any(bad) != 0;
+    if (lane == 0) out.nopen = bad ? ~0u : n;
+    if (!bad && lane < nc && rank < k) {
+      out.id[rank] = e;
+      out.lg[rank] = out.val[e];
+    }
+  }
+  __syncthreads();
+  return out.nopen != ~0u;
 }
 
 // The exact path (every thread of the workgroup; out.id/lg/bd hold the
 // device ranking). Rewrites out.id and out.lg; returns whether every expert
 // was recomputed. out.nneartie gets the adjacent pairs that sent it to the
 // full recompute (near ties with the higher id first).
-template <int PER, bool DEEP>
+template <int PER, bool CLUSTERS>
 __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[PER], const float (&b)[PER],
                              Selection<PER>& out, float mx) {
   const uint32_t E = rv.expert_count, k = rv.top_k;
@@ -675,7 +938,14 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
   // (stable since the certificate's barrier).
   float th = INFINITY;
   for (uint32_t i = 0; i < k; ++i) th = fminf(th, out.lg[i] - kBoundSlack * out.bd[i]);
-  const float scale = rv.rms ? exact_rms_scale<PER>(rv, t, out) : 1.0f;
+  // Far below the maximum the general form ranks by the probabilities themselves.
+  // (CLUSTERS = false: gate/up of several tokens, whose selection is repeated
+  // by every workgroup and wants three wavefronts to a SIMD: the clusters' code
+  // takes 194 registers where the rest takes 168, and 4 tokens' sublayers took
+  // 4% longer with it.)
+  [[maybe_unused]] bool clusters = rv.hidden <= kSplitMaxCols && rv.hidden % 128u == 0u && out.lg[k - 1] - mx >= -kUnderflowGap;
+  float scale = 1.0f;
+  bool have_scale = !rv.rms;
   bool full = false;
   float m = -INFINITY;
   for (;;) {
@@ -702,8 +972,23 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
       if (member[j]) out.cl[pos++] = static_cast<uint16_t>(base + j);
     }
     __syncthreads();
+    if constexpr (CLUSTERS) {
+      if (clusters && !full && nc <= kWave) {
+        clusters = false;
+        if (resolve_clusters(rv, t, out, mx, nc)) {
+          if (tid == 0) {
+            out.nneartie = 0u;
+            out.ncand = nc;
+          }
+          __syncthreads();
+          return false;
+        }
+      }
+    }
+    if (!have_scale) scale = exact_rms_scale<PER>(rv, t, out);
+    have_scale = true;
     for (uint32_t first = 0; first < nc; first += kExactRows)
-      exact_logits<PER, DEEP>(rv, t, out, first, nc - first < kExactRows ? nc - first : kExactRows, scale);
+      exact_logits<PER>(rv, t, out, first, nc - first < kExactRows ? nc - first : kExactRows, scale);
     __syncthreads();
     if (!full && nc <= kWave) {
       // Up to 64 candidates: wavefront 0 ranks them in registers (lane i
@@ -983,7 +1268,7 @@ __device__ __forceinline__ void rank_device(const RouteView& rv, const float (&l
 // otherwise, for workgroups that only read their slot's expert). `count`:
 // add this selection to the routing counters now (otherwise
 // count_selection does it later).
-template <int PER, bool DEEP = false>
+template <int PER, bool CLUSTERS = true>
 __device__ __forceinline__ void select_values(const RouteView& rv, uint32_t t, const float (&l)[PER],
                                               const float (&b)[PER], const uint8_t* const (&tab)[PER],
                                               Selection<PER>& out, bool count, bool need_p = true) {
@@ -1050,7 +1335,7 @@ __device__ __forceinline__ void select_values(const RouteView& rv, uint32_t t, c
   OSMD_STAMP(7, timeline_first());
   if (need_p) sum = ((out.red[2][0] + out.red[2][1]) + out.red[2][2]) + out.red[2][3];
   bool full = false;
-  if (bad) full = select_exact<PER, DEEP>(rv, t, l, b, out, mx);
+  if (bad) full = select_exact<PER, CLUSTERS>(rv, t, l, b, out, mx);
   if (need_p && tid < k) out.p[tid] = expf(out.lg[tid] - mx) / sum;
   if (tid == 0) out.flags = (bad ? 1u : 0u) | (full ? 2u : 0u);
   if (count && tid == 0 && rv.stats != nullptr) {
@@ -1083,7 +1368,7 @@ constexpr uint32_t kMaxPlanes = 8;
 // PLANES = false: the logits are final (the per-token router's), so the
 // router GEMM's plane sums are not compiled in and the loads below are the
 // first thing the workgroup issues.
-template <int PER, bool DEEP = false, bool PLANES = true>
+template <int PER, bool PLANES = true, bool CLUSTERS = true>
 __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Selection<PER>& out, bool count,
                                              bool need_p = true) {
   const uint32_t E = rv.expert_count;
@@ -1179,7 +1464,7 @@ __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Se
     }
     rv.gate_out[t] = 1.0f / (1.0f + expf(-g));  // reference_ops.cpp:214-216
   }
-  select_values<PER, DEEP>(rv, t, p, bnd, tab, out, count, need_p);
+  select_values<PER, CLUSTERS>(rv, t, p, bnd, tab, out, count, need_p);
 }
 
 template <int PER>
@@ -1216,7 +1501,7 @@ __device__ __forceinline__ void publish_selection(const RouteView& rv, uint32_t 
 template <int PER>
 __global__ __launch_bounds__(kSelThreads) void select_kernel(RouteView rv) {
   __shared__ Selection<PER> sel;
-  select_block<PER, true>(rv, blockIdx.x, sel, true);
+  select_block<PER>(rv, blockIdx.x, sel, true);
   publish_selection(rv, blockIdx.x, threadIdx.x, sel);
 }
 
@@ -1543,7 +1828,7 @@ __global__ __launch_bounds__(256) void gate_up_kernel(GateUpParams p) {
       // forms the probabilities.
       const bool publisher = blockIdx.x == 0 && j == 0;
       OSMD_STAMP(4, timeline_first());
-      select_block<PER, false, false>(rv, t, sel, false, publisher);
+      select_block<PER, false, ROWS == kGuRowsOneToken>(rv, t, sel, false, publisher);
       OSMD_STAMP(8, timeline_first());
       rows(pick_blob(rv, sel, j));
       OSMD_STAMP(10, timeline_first());
