@@ -28,6 +28,8 @@
 // one-workgroup-per-token select kernel runs after route_kernel instead, the
 // host reads the ids and writes the slot pointers, and gate_up_kernel reads
 // those.
+#include <type_traits>
+
 #include "device_common.hpp"
 
 namespace {
@@ -814,14 +816,197 @@ __device__ void exact_logits_rd(const RouteView& rv, uint32_t t, Selection<PER>&
   if (tid < nr) out.ex[out.cl[first + tid]] = acc;
 }
 
-template <int PER>
+// The same logits with the loads two steps ahead: router elements in two
+// register sets used on alternate steps, inputs loaded two steps before they
+// are staged, and additions in batches of 64. For the selection kernel (one
+// workgroup per token, registers to spare): a step is then the addition chain
+// rather than the producers' wait for their loads.
+template <int RD, int PER>
+__device__ void exact_logits_deep(const RouteView& rv, uint32_t t, Selection<PER>& out, uint32_t first, uint32_t nr,
+                                  float scale) {
+#pragma clang fp contract(off)
+  const uint32_t D = rv.hidden, tid = threadIdx.x;
+  const bool producer = tid >= kWave;
+  const uint32_t ptid = producer ? tid - kWave : 0u;
+  const uint32_t r = ptid % kExactRows, seg = (ptid / kExactRows) * 16u;
+  const bool active = producer && r < nr;
+  const uint32_t e = r < nr ? out.cl[first + r] : out.cl[first];
+  Q8Row qr{};
+  const uint8_t* row = nullptr;
+  if constexpr (RD == OSM_ROUTER_AFFINE_Q8)
+    qr = q8_row(rv.router, rv.expert_count, e, D, rv.router_group);
+  else
+    row = static_cast<const uint8_t*>(rv.router) + static_cast<size_t>(e) * D * (RD == OSM_META_F32 ? 4u : 2u);
+  struct W16 {
+    Raw8<RD> lo, hi;
+  };
+  struct X1 {
+    uint32_t x;  // as loaded (load_x1_bits)
+    float nw;
+  };
+  auto fetch_w = [&](W16& w, uint32_t chunk) {
+    const uint32_t c = chunk * kExactCols + seg;
+    if (!active) return;
+    if (c < D) {
+      if constexpr (RD == OSM_ROUTER_AFFINE_Q8) load_q8x8(qr, c, w.lo); else load_raw8<RD>(row, c, w.lo);
+    }
+    if (c + 8u < D) {
+      if constexpr (RD == OSM_ROUTER_AFFINE_Q8) load_q8x8(qr, c + 8u, w.hi); else load_raw8<RD>(row, c + 8u, w.hi);
+    }
+  };
+  auto fetch_x = [&](X1& v, uint32_t chunk) {
+    if (!producer) return;
+    const uint32_t c = chunk * kExactCols + ptid;
+    v.x = load_x1_bits(rv, t, c);
+    v.nw = (rv.rms && c < D) ? ldg<float>(rv.norm_weight + c) : 1.0f;
+  };
+  auto stage_x = [&](const X1& v, uint32_t buf) {
+    if (!producer) return;
+    const float xv = x1_value(rv, v.x);
+    out.xe[buf][ptid] = rv.rms ? xv * (scale * v.nw) : xv;
+  };
+  const uint32_t nchunks = (D + kExactCols - 1u) / kExactCols;
+  float acc = 0.0f;
+  // Step k: products of chunk k from w (loaded in step k - 2), w refilled
+  // with chunk k + 2; chunk k + 1's inputs staged from xs (loaded in step
+  // k - 2), xs refilled with chunk k + 3; lane r of wavefront 0 adds chunk
+  // k - 1.
+  auto step = [&](uint32_t k, W16& w, X1& xs) {
+    if (active && k < nchunks) {
+      float4* dst = reinterpret_cast<float4*>(&out.prod[k & 1u][r][seg]);
+      const float4* xe = reinterpret_cast<const float4*>(&out.xe[k & 1u][seg]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 x4 = xe[j];
+        const Raw8<RD>& h = j < 2 ? w.lo : w.hi;
+        const int o = 4 * (j % 2);
+        dst[j] = make_float4(raw8_get<RD>(h, o) * x4.x, raw8_get<RD>(h, o + 1) * x4.y,
+                             raw8_get<RD>(h, o + 2) * x4.z, raw8_get<RD>(h, o + 3) * x4.w);
+      }
+      if (k + 2u < nchunks) fetch_w(w, k + 2u);
+    }
+    if (k + 1u < nchunks) {
+      stage_x(xs, (k + 1u) & 1u);
+      if (k + 3u < nchunks) fetch_x(xs, k + 3u);
+    }
+    if (tid < nr && k > 0u) {
+      const uint32_t c0 = (k - 1u) * kExactCols;
+      acc = chain_sum<16>(out.prod[(k - 1u) & 1u][tid], D - c0 < kExactCols ? D - c0 : kExactCols, acc);
+    }
+    __syncthreads();
+  };
+  W16 wa{}, wb{};
+  X1 xa{}, xb{};
+  fetch_x(xa, 0);
+  fetch_w(wa, 0);
+  if (nchunks > 1u) fetch_w(wb, 1);
+  stage_x(xa, 0);
+  if (nchunks > 1u) fetch_x(xb, 1);
+  if (nchunks > 2u) fetch_x(xa, 2);
+  __syncthreads();
+  // The adders' wavefront issues first on its SIMD while it adds: each
+  // addition waits for the one before it, and a wavefront of another
+  // workgroup sharing the SIMD would otherwise take the slots in between.
+  const bool adder_wave = tid < kWave;
+  if (adder_wave) __builtin_amdgcn_s_setprio(2);
+  // Even steps stage odd chunks from xb, odd steps even chunks from xa.
+  for (uint32_t k = 0; k <= nchunks; k += 2u) {
+    step(k, wa, xb);
+    if (k + 1u <= nchunks) step(k + 1u, wb, xa);
+  }
+  if (adder_wave) __builtin_amdgcn_s_setprio(0);
+  if (tid < nr) out.ex[out.cl[first + tid]] = acc;
+}
+
+template <int PER, bool DEEP>
 __device__ void exact_logits(const RouteView& rv, uint32_t t, Selection<PER>& out, uint32_t first, uint32_t nr,
                              float scale) {
+  auto run = [&](auto rd) {
+    if constexpr (DEEP)
+      exact_logits_deep<rd.value>(rv, t, out, first, nr, scale);
+    else
+      exact_logits_rd<rd.value>(rv, t, out, first, nr, scale);
+  };
   switch (rv.router_dtype) {
-    case OSM_META_F32: exact_logits_rd<OSM_META_F32>(rv, t, out, first, nr, scale); break;
-    case OSM_META_F16: exact_logits_rd<OSM_META_F16>(rv, t, out, first, nr, scale); break;
-    case OSM_ROUTER_AFFINE_Q8: exact_logits_rd<OSM_ROUTER_AFFINE_Q8>(rv, t, out, first, nr, scale); break;
-    default: exact_logits_rd<OSM_META_BF16>(rv, t, out, first, nr, scale); break;
+    case OSM_META_F32: run(std::integral_constant<int, OSM_META_F32>{}); break;
+    case OSM_META_F16: run(std::integral_constant<int, OSM_META_F16>{}); break;
+    case OSM_ROUTER_AFFINE_Q8: run(std::integral_constant<int, OSM_ROUTER_AFFINE_Q8>{}); break;
+    default: run(std::integral_constant<int, OSM_META_BF16>{}); break;
+  }
+}
+
+// The reference's logits of every expert for token t, in out.ex (the full
+// recompute): each thread runs the chains of its own PER experts side by side,
+// 8 or 16 columns of a row at a time, over x staged in LDS 2,048 columns at a time.
+// Sixteen experts to a pass of exact_logits, 512 experts took 32 passes, 0.45
+// ms of which a 4,096-token launch, that has one such token in three or four,
+// waited for all.
+template <int RD, int PER>
+__device__ void full_logits_rd(const RouteView& rv, uint32_t t, Selection<PER>& out, float scale) {
+#pragma clang fp contract(off)
+  constexpr uint32_t kStage = 2048;
+  constexpr uint32_t kAhead = PER <= 2 ? 2u : 1u;  // 8-column words of each row loaded together
+  static_assert(kStage <= 2u * kExactRows * kExactStride, "the staged input fits the product buffer");
+  const uint32_t D = rv.hidden, E = rv.expert_count, base = threadIdx.x * PER;
+  float* stage = &out.prod[0][0][0];
+  float acc[PER];
+  const uint8_t* row[PER];
+  Q8Row qr[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    acc[j] = 0.0f;
+    const uint32_t e = base + j < E ? base + j : E - 1u;
+    if constexpr (RD == OSM_ROUTER_AFFINE_Q8)
+      qr[j] = q8_row(rv.router, E, e, D, rv.router_group);
+    else
+      row[j] = static_cast<const uint8_t*>(rv.router) + static_cast<size_t>(e) * D * (RD == OSM_META_F32 ? 4u : 2u);
+  }
+  for (uint32_t c0 = 0; c0 < D; c0 += kStage) {
+    const uint32_t n = D - c0 < kStage ? D - c0 : kStage;  // a multiple of 32
+    __syncthreads();  // the buffer is free
+    for (uint32_t i = threadIdx.x; i < n; i += kSelThreads) {
+      const float v = load_x1(rv, t, c0 + i);
+      stage[i] = rv.rms ? v * (scale * ldg<float>(rv.norm_weight + c0 + i)) : v;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t c = 0; c < n; c += 8u * kAhead) {
+      Raw8<RD> w[PER][kAhead];
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+#pragma unroll
+        for (uint32_t u = 0; u < kAhead; ++u) {
+          if constexpr (RD == OSM_ROUTER_AFFINE_Q8)
+            load_q8x8(qr[j], c0 + c + 8u * u, w[j][u]);
+          else
+            load_raw8<RD>(row[j], c0 + c + 8u * u, w[j][u]);
+        }
+#pragma unroll
+      for (uint32_t u = 0; u < kAhead; ++u) {
+        const float4 xa = *reinterpret_cast<const float4*>(stage + c + 8u * u);
+        const float4 xb = *reinterpret_cast<const float4*>(stage + c + 8u * u + 4u);
+        const float x[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int j = 0; j < PER; ++j) {
+            const float prod = raw8_get<RD>(w[j][u], i) * x[i];
+            acc[j] = acc[j] + prod;
+          }
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (base + j < E) out.ex[base + j] = acc[j];
+}
+template <int PER>
+__device__ void full_logits(const RouteView& rv, uint32_t t, Selection<PER>& out, float scale) {
+  switch (rv.router_dtype) {
+    case OSM_META_F32: full_logits_rd<OSM_META_F32>(rv, t, out, scale); break;
+    case OSM_META_F16: full_logits_rd<OSM_META_F16>(rv, t, out, scale); break;
+    case OSM_ROUTER_AFFINE_Q8: full_logits_rd<OSM_ROUTER_AFFINE_Q8>(rv, t, out, scale); break;
+    default: full_logits_rd<OSM_META_BF16>(rv, t, out, scale); break;
   }
 }
 
@@ -928,7 +1113,21 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
 // device ranking). Rewrites out.id and out.lg; returns whether every expert
 // was recomputed. out.nneartie gets the adjacent pairs that sent it to the
 // full recompute (near ties with the higher id first).
-template <int PER, bool CLUSTERS>
+// How a kernel's selection takes the exact path: kExactPlain the general form
+// alone (gate/up of several tokens, whose selection every workgroup repeats and
+// which wants three wavefronts to a SIMD: the clusters' code takes 194
+// registers where the rest takes 168, and 4 tokens' sublayers took 4% longer
+// with it); kExactClusters open clusters first, and the full recompute by
+// full_logits; kExactDeep the general form with its loads two steps ahead (253
+// registers: either of the other two beside it spills or halves the
+// occupancy). The selection kernel takes clusters in the sublayer form, where
+// they also split the RMS scale's chain (64 tokens: 35 -> 29 µs a launch), and
+// from 1,024 tokens on, where one launch in three or four holds a full recompute
+// (4,096 tokens, two layers: 2,699 -> 2,627 µs). Otherwise the deep form:
+// behind the router GEMM's wider bounds the slowest token of a 512-token launch
+// has four open experts or more, two passes and up (29 µs a launch against 25).
+enum ExactMode : int { kExactPlain = 0, kExactClusters = 1, kExactDeep = 2 };
+template <int PER, ExactMode MODE>
 __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[PER], const float (&b)[PER],
                              Selection<PER>& out, float mx) {
   const uint32_t E = rv.expert_count, k = rv.top_k;
@@ -939,10 +1138,6 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
   float th = INFINITY;
   for (uint32_t i = 0; i < k; ++i) th = fminf(th, out.lg[i] - kBoundSlack * out.bd[i]);
   // Far below the maximum the general form ranks by the probabilities themselves.
-  // (CLUSTERS = false: gate/up of several tokens, whose selection is repeated
-  // by every workgroup and wants three wavefronts to a SIMD: the clusters' code
-  // takes 194 registers where the rest takes 168, and 4 tokens' sublayers took
-  // 4% longer with it.)
   [[maybe_unused]] bool clusters = rv.hidden <= kSplitMaxCols && rv.hidden % 128u == 0u && out.lg[k - 1] - mx >= -kUnderflowGap;
   float scale = 1.0f;
   bool have_scale = !rv.rms;
@@ -972,7 +1167,7 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
       if (member[j]) out.cl[pos++] = static_cast<uint16_t>(base + j);
     }
     __syncthreads();
-    if constexpr (CLUSTERS) {
+    if constexpr (MODE == kExactClusters) {
       if (clusters && !full && nc <= kWave) {
         clusters = false;
         if (resolve_clusters(rv, t, out, mx, nc)) {
@@ -987,8 +1182,12 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
     }
     if (!have_scale) scale = exact_rms_scale<PER>(rv, t, out);
     have_scale = true;
-    for (uint32_t first = 0; first < nc; first += kExactRows)
-      exact_logits<PER>(rv, t, out, first, nc - first < kExactRows ? nc - first : kExactRows, scale);
+    if (MODE == kExactClusters && full) {  // every expert is a candidate
+      if constexpr (MODE == kExactClusters) full_logits<PER>(rv, t, out, scale);
+    } else {
+      for (uint32_t first = 0; first < nc; first += kExactRows)
+        exact_logits<PER, MODE == kExactDeep>(rv, t, out, first, nc - first < kExactRows ? nc - first : kExactRows, scale);
+    }
     __syncthreads();
     if (!full && nc <= kWave) {
       // Up to 64 candidates: wavefront 0 ranks them in registers (lane i
@@ -1268,7 +1467,7 @@ __device__ __forceinline__ void rank_device(const RouteView& rv, const float (&l
 // otherwise, for workgroups that only read their slot's expert). `count`:
 // add this selection to the routing counters now (otherwise
 // count_selection does it later).
-template <int PER, bool CLUSTERS = true>
+template <int PER, ExactMode MODE>
 __device__ __forceinline__ void select_values(const RouteView& rv, uint32_t t, const float (&l)[PER],
                                               const float (&b)[PER], const uint8_t* const (&tab)[PER],
                                               Selection<PER>& out, bool count, bool need_p = true) {
@@ -1335,7 +1534,7 @@ __device__ __forceinline__ void select_values(const RouteView& rv, uint32_t t, c
   OSMD_STAMP(7, timeline_first());
   if (need_p) sum = ((out.red[2][0] + out.red[2][1]) + out.red[2][2]) + out.red[2][3];
   bool full = false;
-  if (bad) full = select_exact<PER, CLUSTERS>(rv, t, l, b, out, mx);
+  if (bad) full = select_exact<PER, MODE>(rv, t, l, b, out, mx);
   if (need_p && tid < k) out.p[tid] = expf(out.lg[tid] - mx) / sum;
   if (tid == 0) out.flags = (bad ? 1u : 0u) | (full ? 2u : 0u);
   if (count && tid == 0 && rv.stats != nullptr) {
@@ -1368,7 +1567,7 @@ constexpr uint32_t kMaxPlanes = 8;
 // PLANES = false: the logits are final (the per-token router's), so the
 // router GEMM's plane sums are not compiled in and the loads below are the
 // first thing the workgroup issues.
-template <int PER, bool PLANES = true, bool CLUSTERS = true>
+template <int PER, bool PLANES, ExactMode MODE>
 __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Selection<PER>& out, bool count,
                                              bool need_p = true) {
   const uint32_t E = rv.expert_count;
@@ -1464,7 +1663,7 @@ __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Se
     }
     rv.gate_out[t] = 1.0f / (1.0f + expf(-g));  // reference_ops.cpp:214-216
   }
-  select_values<PER, CLUSTERS>(rv, t, p, bnd, tab, out, count, need_p);
+  select_values<PER, MODE>(rv, t, p, bnd, tab, out, count, need_p);
 }
 
 template <int PER>
@@ -1498,10 +1697,10 @@ __device__ __forceinline__ void publish_selection(const RouteView& rv, uint32_t 
   if (tid == 0) rv.mass[t] = mass;
 }
 
-template <int PER>
+template <int PER, ExactMode MODE>
 __global__ __launch_bounds__(kSelThreads) void select_kernel(RouteView rv) {
   __shared__ Selection<PER> sel;
-  select_block<PER>(rv, blockIdx.x, sel, true);
+  select_block<PER, true, MODE>(rv, blockIdx.x, sel, true);
   publish_selection(rv, blockIdx.x, threadIdx.x, sel);
 }
 
@@ -1828,7 +2027,7 @@ __global__ __launch_bounds__(256) void gate_up_kernel(GateUpParams p) {
       // forms the probabilities.
       const bool publisher = blockIdx.x == 0 && j == 0;
       OSMD_STAMP(4, timeline_first());
-      select_block<PER, false, ROWS == kGuRowsOneToken>(rv, t, sel, false, publisher);
+      select_block<PER, false, ROWS == kGuRowsOneToken ? kExactClusters : kExactPlain>(rv, t, sel, false, publisher);
       OSMD_STAMP(8, timeline_first());
       rows(pick_blob(rv, sel, j));
       OSMD_STAMP(10, timeline_first());
@@ -2480,9 +2679,20 @@ RouteView route_view(const osmd_moe_args& a) {
 
 int launch_select(const osmd_moe_args& a, hipStream_t st) {
   const RouteView rv = route_view(a);
+  const bool clusters = rv.rms != 0u || a.tokens >= 1024u;  // ExactMode
   switch (selection_per(a.expert_count)) {
-    case 2: select_kernel<2><<<a.tokens, kSelThreads, 0, st>>>(rv); break;
-    default: select_kernel<4><<<a.tokens, kSelThreads, 0, st>>>(rv); break;
+    case 2:
+      if (clusters)
+        select_kernel<2, kExactClusters><<<a.tokens, kSelThreads, 0, st>>>(rv);
+      else
+        select_kernel<2, kExactDeep><<<a.tokens, kSelThreads, 0, st>>>(rv);
+      break;
+    default:
+      if (clusters)
+        select_kernel<4, kExactClusters><<<a.tokens, kSelThreads, 0, st>>>(rv);
+      else
+        select_kernel<4, kExactDeep><<<a.tokens, kSelThreads, 0, st>>>(rv);
+      break;
   }
   return launch_status();
 }
