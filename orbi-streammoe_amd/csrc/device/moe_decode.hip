@@ -1138,7 +1138,8 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
   float th = INFINITY;
   for (uint32_t i = 0; i < k; ++i) th = fminf(th, out.lg[i] - kBoundSlack * out.bd[i]);
   // Far below the maximum the general form ranks by the probabilities themselves.
-  [[maybe_unused]] bool clusters = rv.hidden <= kSplitMaxCols && rv.hidden % 128u == 0u && out.lg[k - 1] - mx >= -kUnderflowGap;
+  [[maybe_unused]] bool clusters = MODE == kExactClusters && rv.hidden <= kSplitMaxCols && rv.hidden % 128u == 0u &&
+                                   out.lg[k - 1] - mx >= -kUnderflowGap;
   float scale = 1.0f;
   bool have_scale = !rv.rms;
   bool full = false;
@@ -1699,6 +1700,7 @@ __device__ __forceinline__ void publish_selection(const RouteView& rv, uint32_t 
 
 template <int PER, ExactMode MODE>
 __global__ __launch_bounds__(kSelThreads) void select_kernel(RouteView rv) {
+  if constexpr (MODE == kExactDeep) rv.rms = 0u;  // launched without it alone: nothing of the norm is compiled in
   __shared__ Selection<PER> sel;
   select_block<PER, true, MODE>(rv, blockIdx.x, sel, true);
   publish_selection(rv, blockIdx.x, threadIdx.x, sel);
