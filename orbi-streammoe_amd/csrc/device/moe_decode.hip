@@ -1018,9 +1018,11 @@ __device__ void full_logits(const RouteView& rv, uint32_t t, Selection<PER>& out
 // the order within. Between cuts lie clusters: one of a single expert is in
 // its place; the reference's logits of the others, if they are at most
 // kMaxOpen and reach the first k ranks, are summed as it sums them, and order
-// their cluster: by the logit, equal ones by id. Two neighbours of different
-// logit whose lower one has the lower id must be apart by the tie margin, or
-// their probabilities might be equal. True when out.id and out.lg are then the
+// their cluster: by the logit, equal ones by id. Every lower logit of a lower
+// id in the cluster, whatever its own rank, must be apart from one of the first
+// k ranks by the tie margin, or their probabilities might be equal and the
+// lower id come first (with ids 20, 30 and 10 around rank k, 20 and 30 in order
+// say nothing about 20 and 10). True when out.id and out.lg are then the
 // reference's; false (nothing written) where the general form below is needed.
 // Every thread of the workgroup calls it.
 template <int PER>
@@ -1080,23 +1082,18 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
     if (open) {
       const float v = out.uval[upos];
       rank = start;
-      float nv = -INFINITY;  // the next lower of the cluster
-      uint32_t ne = 0u;
+      bool tied = false;  // a lower logit of a lower id whose probability might be equal
 #pragma unroll 1
       for (uint32_t i = 0; i < n; ++i) {
         if (out.ustart[i] != start || i == upos) continue;
         const float w = out.uval[i];
         const uint32_t ei = out.uid[i];
-        const bool above = w > v || (w == v && ei < e);
-        if (above) {
+        if (w > v || (w == v && ei < e))
           ++rank;
-        } else if (w > nv || (w == nv && ei < ne)) {
-          nv = w;
-          ne = ei;
-        }
+        else
+          tied |= ei < e && !(v - w > tie_margin(mx, w));
       }
-      bad = !(v - v == 0.0f) ||
-            (rank < k && nv > -INFINITY && v != nv && e > ne && !(v - nv > tie_margin(mx, nv)));
+      bad = !(v - v == 0.0f) || (rank < k && tied);
     }
     bad = __any(bad) != 0;
     if (lane == 0) out.nopen = bad ? ~0u : n;

@@ -49,3 +49,77 @@ def test_routing_clusters(ctx, D, clusters):
             moe.decode_device(slab, 0, xd.ptr, yd.ptr, 1, sublayer=sublayer)
             assert np.array_equal(moe.routing(1)["ids"][0], want[t]), (sublayer, t)
     assert moe.routing_stats()["exact"] > 0
+
+
+# ---------------------------------------------------------------------------
+# Logits set exactly: the router's input is 1 in its first column and 0
+# elsewhere, so expert e's logit is router[e, 0] in whatever order it is summed.
+# In the sublayer form that input is 16 normalised at 256 columns (the mean of
+# the squares is 1) times a norm weight of 1/16. The bounds do not know that
+# the sums are exact: logits a few units in the last place apart are open.
+
+EXACT_D = 256
+
+
+def rows_for(logits):
+    router = np.zeros((len(logits), EXACT_D), np.float32)
+    router[:, 0] = logits
+    return router
+
+
+def every_selection(ctx, router, k, x=None, sublayers=(False, True)):
+    """(label, ids, stats) of each kernel that selects: one token and four (inside gate/up), 16 (the selection kernel
+    behind the per-token router), 48 (behind the router GEMM), with and without the norm, and 1,024 bf16 tokens."""
+    E, D = router.shape
+    I, G = 128, 64
+    g = osm_hip.geometry(D, I, G, osm_hip.BF16)
+    slab = osm_hip.ExpertSlab(ctx, g, 1, E)
+    slab.synthesize(1)
+    nw = np.full(D, 1 / 16, np.float32)
+    moe = osm_hip.MoeLayer(ctx, g, E, k, router, osm_hip.F32, None, nw, None, max_tokens=1024, rms_eps=1e-20)
+    if x is None:
+        x = np.zeros(D, np.float32)
+        x[0] = 1.0
+    for sublayer in sublayers:
+        xin = 16 * x if sublayer else x
+        if sublayer:
+            assert np.array_equal(O.rms_norm(xin, 1, D, nw, 1e-20), x)
+        for T, path in ((1, osm_hip.PATH_PER_TOKEN), (4, osm_hip.PATH_PER_TOKEN), (16, osm_hip.PATH_PER_TOKEN),
+                        (48, osm_hip.PATH_GROUPED)):
+            moe.set_path(path)
+            xd, yd = ctx.alloc(T * D * 4), ctx.alloc(T * D * 4)
+            xd.upload(np.tile(xin, (T, 1)))
+            moe.routing_stats(reset=True)
+            moe.decode_device(slab, 0, xd.ptr, yd.ptr, T, sublayer=sublayer)
+            yield (T, sublayer), moe.routing(T)["ids"], moe.routing_stats()
+    T = 1024
+    xd, yd = ctx.alloc(T * D * 2), ctx.alloc(T * D * 4)
+    xd.upload(np.tile((x.view(np.uint32) >> 16).astype(np.uint16), (T, 1)))  # x is bf16 already
+    moe.routing_stats(reset=True)
+    moe.prefill_device(slab, 0, xd.ptr, yd.ptr, T)
+    yield (T, "prefill"), moe.routing(T)["ids"], moe.routing_stats()
+
+
+def check_every_selection(ctx, logits, k):
+    router = rows_for(logits)
+    x = np.zeros(EXACT_D, np.float32)
+    x[0] = 1.0
+    want = O.route_qwen_top_k(x, router, EXACT_D, len(logits), k, True)["ids"]
+    for label, ids, _ in every_selection(ctx, router, k):
+        assert np.array_equal(ids, np.tile(want, (len(ids), 1))), (label, ids[0], want)
+    return list(want)
+
+
+def distant(E=40):
+    return np.full(E, -5, np.float32)
+
+
+# Three experts whose logits, 7 below the largest, differ by less than the rounding of that distance: one probability,
+# so the reference takes id 10, the lowest logit of the three (or the three in id order). Ranked by the logit, 20 and
+# 30 are the neighbours across the end of the picks, in id order themselves.
+@pytest.mark.parametrize("k,want", [(2, [0, 10]), (3, [0, 10, 20]), (4, [0, 10, 20, 30])])
+@pytest.mark.parametrize("l30", [1 + 2.0**-23, 1 + 2.0**-22])
+def test_one_probability_across_the_picks(ctx, k, want, l30):
+    logits = distant()
+    logits[0], logits[20], logits[30], logits[10] = 8, 1 + 2.0**-22, l30, 1
+    assert check_every_selection(ctx, logits, k) == want
