@@ -347,9 +347,9 @@ int osm_moe_layer_routing(osm_context ctx, osm_moe_layer l, uint32_t tokens,
  * per token per call), out[1] selections that took that exact path, out[2]
  * exact paths that recomputed every expert and ranked them by the
  * reference's own probabilities (picks near exp underflow, or a near tie),
- * out[3] the near ties that sent a selection there: adjacent candidates
- * whose exps (the host libm's bits) are close enough for their
- * probabilities to round to one value, with the higher id ranked first.
+ * out[3] the near ties that sent a selection there: picks with a lower
+ * candidate of a lower id whose exp (the host libm's bits) is close enough
+ * for their probabilities to round to one value.
  * Synchronises the context's stream; reset != 0 zeroes them afterwards. */
 int osm_moe_layer_routing_stats(osm_context ctx, osm_moe_layer l, uint32_t out[4], int reset);
 

@@ -266,8 +266,9 @@ __device__ __forceinline__ float raw8_get(const Raw8<RD>& r, int j) {
 // in id order; p orders as e does, except that two different e can round to
 // one p, and then the lower id wins. That can only happen for e_a > e_c
 // within 2^-22 e_a (one ulp of the quotient, or 2^-138 where the quotient is
-// subnormal). When such a pair is adjacent among the first k + 1 candidates
-// with the higher id first, and whenever the k-th candidate is more than 80
+// subnormal). When one of the first k candidates is that close to a lower one
+// of a lower id, next to it or not (others of its own e may lie between), and
+// whenever the k-th candidate is more than 80
 // below m (exps near or at underflow), every expert is recomputed: S is then
 // summed as the reference sums it and the experts are ranked by fl(e / S),
 // ties to the lower id, which is the reference's ranking itself.
@@ -1108,8 +1109,8 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
 
 // The exact path (every thread of the workgroup; out.id/lg/bd hold the
 // device ranking). Rewrites out.id and out.lg; returns whether every expert
-// was recomputed. out.nneartie gets the adjacent pairs that sent it to the
-// full recompute (near ties with the higher id first).
+// was recomputed. out.nneartie gets the picks that sent it to the full
+// recompute (near ties with a lower id behind them).
 // How a kernel's selection takes the exact path: kExactPlain the general form
 // alone (gate/up of several tokens, whose selection every workgroup repeats and
 // which wants three wavefronts to a SIMD: the clusters' code takes 194
@@ -1200,24 +1201,15 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
         const float key = act ? osm_libm_expf(x - mm) : -1.0f;
         if (act) out.aux[e] = key;
         uint32_t rk = 0u;
+        bool near = false;  // a lower candidate of a lower id whose quotient might be equal
         for (uint32_t i = 0; i < nc; ++i) {
           const float w = readlane_f(key, static_cast<int>(i));
           const uint32_t ei = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(e), static_cast<int>(i)));
           rk += (w > key || (w == key && ei < e)) ? 1u : 0u;
+          near |= w < key && ei < e && key - w <= 0x1p-22f * key + 0x1p-138f;
         }
         if (act && rk <= k) out.fid[rk] = e;
-        // This candidate (rank rk) against the one ranked rk + 1.
-        const uint32_t n = nc < k + 1u ? nc : k + 1u;
-        float ec = 0.0f;
-        uint32_t c = 0u;
-        for (uint32_t i = 0; i < nc; ++i) {
-          const uint32_t ri = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(rk), static_cast<int>(i)));
-          if (ri == rk + 1u) {
-            ec = readlane_f(key, static_cast<int>(i));
-            c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(e), static_cast<int>(i)));
-          }
-        }
-        const bool near = act && rk + 1u < n && e > c && key != ec && key - ec <= 0x1p-22f * key + 0x1p-138f;
+        near = act && rk < k && near;
         const uint64_t nb = __ballot(near);
         const uint64_t kb = __ballot(act && rk == k - 1u);  // one lane: nc >= k (the picks are candidates)
         const float xk = readlane_f(x, static_cast<int>(__builtin_ctzll(kb)));
@@ -1270,49 +1262,46 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
         if (member[j]) key[j] = __fdiv_rn(key[j], S);
     }
     // Ranking keys in list order in ckey (the products' buffer is free now),
-    // so that the ranking reads them without an indirection.
+    // so that the ranking reads them without an indirection. A pick and a lower
+    // candidate of a lower id whose e are close enough for their quotients by S
+    // to round to one p (the reference would put the lower id first) are a near
+    // tie, whatever lies between them.
     float* ckey = &out.prod[0][0][0];
 #pragma unroll
     for (int j = 0; j < PER; ++j)
       if (member[j]) ckey[cpos[j]] = key[j];
     __syncthreads();
+    uint32_t nnear = 0u;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      if (!member[j]) continue;
-      const uint32_t e = base + j;
-      const float v = key[j];
-      uint32_t rk = 0;
+      bool near = false;
+      if (member[j]) {
+        const uint32_t e = base + j;
+        const float v = key[j];
+        uint32_t rk = 0;
 #pragma unroll 4
-      for (uint32_t i = 0; i < nc; ++i) {
-        const float w = ckey[i];
-        rk += (w > v || (w == v && out.cl[i] < e)) ? 1u : 0u;
+        for (uint32_t i = 0; i < nc; ++i) {
+          const float w = ckey[i];
+          const bool lower_id = out.cl[i] < e;
+          rk += (w > v || (w == v && lower_id)) ? 1u : 0u;
+          near |= w < v && lower_id && v - w <= 0x1p-22f * v + 0x1p-138f;
+        }
+        if (rk <= k) out.fid[rk] = e;
+        near = near && rk < k;
       }
-      if (rk <= k) out.fid[rk] = e;
+      nnear += static_cast<uint32_t>(__popcll(__ballot(near)));
     }
+    if (lane == 0) out.wcount[wave] = nnear;  // the counts of the list are read
     __syncthreads();
     if (full) {
       if (tid == 0) out.ncand = nc;
       break;
     }
-    // Adjacent candidates among the first k + 1 (there are at least k: the
-    // device's picks are candidates), one pair per lane: a pair ranked with
-    // the higher id first whose e are close enough for their quotients by S
-    // to round to one p, where the reference would put the lower id first.
-    if (tid < kWave) {
-      const uint32_t n = nc < k + 1u ? nc : k + 1u;
-      bool near = false;
-      if (lane + 1u < n) {
-        const uint32_t a = out.fid[lane], c = out.fid[lane + 1u];
-        const float ea = out.aux[a], ec = out.aux[c];  // ea >= ec (ranked)
-        near = a > c && ea != ec && ea - ec <= 0x1p-22f * ea + 0x1p-138f;
-      }
-      const uint32_t count = static_cast<uint32_t>(__popcll(__ballot(near)));
-      if (lane == 0) out.nneartie = count;
-    }
-    __syncthreads();
-    // Such a pair, or exps near underflow beyond 80 below m: rank every
+    nnear = out.wcount[0] + out.wcount[1] + out.wcount[2] + out.wcount[3];
+    if (tid == 0) out.nneartie = nnear;
+    // A near tie, or exps near underflow beyond 80 below m: rank every
     // expert by the reference's probabilities.
-    const bool again = out.nneartie != 0u || !(out.ex[out.fid[k - 1]] - m >= -kUnderflowGap);
+    const bool again = nnear != 0u || !(out.ex[out.fid[k - 1]] - m >= -kUnderflowGap);
     if (!again) {
       if (tid == 0) out.ncand = nc;
       break;

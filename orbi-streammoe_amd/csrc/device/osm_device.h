@@ -165,8 +165,8 @@ typedef struct osmd_moe_args {
    * otherwise recomputes the candidates' logits in the reference's order from
    * x (fp32, or bf16 when x_bf16; RMS-normalised first in the sublayer form).
    * route_stats (null, or 4 counters, added to): selections, selections that
-   * took the exact path, exact paths that ranked every expert, and adjacent
-   * picks whose order rests on exp rounding within 5 ulps. */
+   * took the exact path, exact paths that ranked every expert, and picks whose
+   * probability a lower logit of a lower id might equal. */
   float* logit_bounds;
   const float* bound_planes;
   uint32_t* route_stats;

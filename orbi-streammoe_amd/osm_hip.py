@@ -754,10 +754,10 @@ class MoeLayer(_Handle):
 
     def routing_stats(self, reset=False) -> dict:
         """Selections, those that took the exact path, exact paths over every
-        expert, and the adjacent near ties (exps close enough for their
-        probabilities to round to one value, the higher id first) that sent a
-        selection to the recompute over every expert, since creation or a
-        reset."""
+        expert, and the near ties (picks with a lower candidate of a lower id
+        whose exps are close enough for their probabilities to round to one
+        value) that sent a selection to the recompute over every expert, since
+        creation or a reset."""
         v = (c_uint32 * 4)()
         check(load().osm_moe_layer_routing_stats(self.ctx.h, self.h, v, 1 if reset else 0))
         return dict(zip(("selections", "exact", "exact_all", "near_ties"), list(v)))

@@ -7,6 +7,7 @@ import pytest
 
 import oracle as O
 import osm_hip
+from test_gpu_routing_exact import _libm_expf, _softmax_sum
 
 pytestmark = pytest.mark.gpu
 
@@ -123,3 +124,32 @@ def test_one_probability_across_the_picks(ctx, k, want, l30):
     logits = distant()
     logits[0], logits[20], logits[30], logits[10] = 8, 1 + 2.0**-22, l30, 1
     assert check_every_selection(ctx, logits, k) == want
+
+
+def quotient_tie(extra):
+    """(logits, want): 20 and 30 share a logit, 10's exp is one unit below theirs and divides by the softmax sum to the
+    same probability; `extra` more experts are within the bounds' reach, too far for a tie."""
+    expf = _libm_expf()
+    rng = np.random.default_rng(3)
+    E = 40 + extra
+    f = np.float32
+    while True:
+        logits = (-1 - 2 * rng.random(E)).astype(np.float32)
+        logits[0] = 1
+        a = f(0.15 + 0.2 * rng.random())
+        b = f(a - f(2.0**-24))
+        ea, eb = expf(f(a - 1)), expf(f(b - 1))
+        if eb == ea or np.nextafter(eb, f(1)) != ea:
+            continue
+        logits[20], logits[30], logits[10] = a, a, b
+        for j in range(extra):
+            logits[40 + j] = a - f(1e-6) * f(1 + j % 8)
+        if f(ea / _softmax_sum(logits, expf)) == f(eb / _softmax_sum(logits, expf)):
+            return logits
+
+
+# The two of one exp are the neighbours across the end of the picks; the reference picks 10. Up to 64 candidates are
+# ranked in one wavefront's registers, more in LDS.
+@pytest.mark.parametrize("extra", [0, 70])
+def test_quotient_tie_behind_an_equal_exp(ctx, extra):
+    assert check_every_selection(ctx, quotient_tie(extra), 2) == [0, 10]
