@@ -245,13 +245,13 @@ __device__ __forceinline__ float raw8_get(const Raw8<RD>& r, int j) {
 //  - adjacent picks i, i+1: l_i - l_{i+1} > s (b_i + b_{i+1}), plus kappa
 //    when the lower logit has the lower id;
 //  - every expert e outside the picks: l_e + s b_e + kappa(e) < l_k - s b_k;
-//  - the k-th pick within 80 of the largest logit.
+//  - the k-th pick's lower bound within 80 of the largest's upper bound.
 //
 // s = 1 + 2^-9 covers a common factor 1 + eta by which the device's
 // RMS-normalised input can differ from the reference's (eta <= n u for a
 // width n <= 8192 and u = 2^-24, from the two sums of squares) and the
 // rounding of the bounds themselves. kappa = 2^-20 + 2^-23 (m - l + 1), m
-// the largest logit: a gap in L larger than that keeps the two
+// the largest upper bound (the reference's largest logit is no higher): a gap in L larger than that keeps the two
 // probabilities exp(fl(L - m)) / S at least four ulps apart whatever the
 // rounding of the subtraction, the exp (within one ulp) and the division, so
 // the reference's probabilities cannot tie where the device's logits do not.
@@ -1027,7 +1027,7 @@ __device__ void full_logits(const RouteView& rv, uint32_t t, Selection<PER>& out
 // reference's; false (nothing written) where the general form below is needed.
 // Every thread of the workgroup calls it.
 template <int PER>
-__device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>& out, float mx, uint32_t nc) {
+__device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>& out, uint32_t nc) {
   const uint32_t k = rv.top_k, tid = threadIdx.x, lane = tid % kWave;
   uint32_t e = 0u, start = 0u, upos = 0u;
   bool open = false;
@@ -1052,7 +1052,8 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
       l = out.val[e];
       b = out.aux[e];
     }
-    const float lo = l - kBoundSlack * b, hi = l + kBoundSlack * b + tie_margin(mx, l);
+    const float top = wave_max(l + kBoundSlack * b);  // the largest logit of all is a candidate's
+    const float lo = l - kBoundSlack * b, hi = l + kBoundSlack * b + tie_margin(top, l);
     float low = INFINITY, high = -INFINITY;
 #pragma unroll 1
     for (uint32_t i = 0; i < nc; ++i) {
@@ -1080,6 +1081,12 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
   if (tid < kWave) {
     uint32_t rank = lane;
     bool bad = false;
+    // The reference's logits, or what bounds them: exps near or at underflow
+    // tie where the logits do not, so far below the largest the general form
+    // ranks by the probabilities themselves.
+    const float l = lane < nc ? out.val[e] : -INFINITY, b = lane < nc ? out.aux[e] : 0.0f;
+    const float top = wave_max(open ? out.uval[upos] : l + kBoundSlack * b);
+    float least = l - kBoundSlack * b;
     if (open) {
       const float v = out.uval[upos];
       rank = start;
@@ -1092,10 +1099,12 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
         if (w > v || (w == v && ei < e))
           ++rank;
         else
-          tied |= ei < e && !(v - w > tie_margin(mx, w));
+          tied |= ei < e && !(v - w > tie_margin(top, w));
       }
       bad = !(v - v == 0.0f) || (rank < k && tied);
+      least = v;
     }
+    bad = bad || (lane < nc && rank < k && !(least - top >= -kUnderflowGap));
     bad = __any(bad) != 0;
     if (lane == 0) out.nopen = bad ? ~0u : n;
     if (!bad && lane < nc && rank < k) {
@@ -1127,38 +1136,51 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
 enum ExactMode : int { kExactPlain = 0, kExactClusters = 1, kExactDeep = 2 };
 template <int PER, ExactMode MODE>
 __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[PER], const float (&b)[PER],
-                             Selection<PER>& out, float mx) {
+                             Selection<PER>& out) {
   const uint32_t E = rv.expert_count, k = rv.top_k;
   const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const uint32_t base = tid * PER;
-  // The picks' lowest lower bound, by every thread from the ranking in LDS
-  // (stable since the certificate's barrier).
-  float th = INFINITY;
-  for (uint32_t i = 0; i < k; ++i) th = fminf(th, out.lg[i] - kBoundSlack * out.bd[i]);
-  // Far below the maximum the general form ranks by the probabilities themselves.
-  [[maybe_unused]] bool clusters = MODE == kExactClusters && rv.hidden <= kSplitMaxCols && rv.hidden % 128u == 0u &&
-                                   out.lg[k - 1] - mx >= -kUnderflowGap;
+  // The picks' lowest lower and highest upper bound, by every thread from the
+  // ranking in LDS (stable since the certificate's barrier).
+  float th = INFINITY, top = -INFINITY;
+  for (uint32_t i = 0; i < k; ++i) {
+    th = fminf(th, out.lg[i] - kBoundSlack * out.bd[i]);
+    top = fmaxf(top, out.lg[i] + kBoundSlack * out.bd[i]);
+  }
+  [[maybe_unused]] bool clusters = MODE == kExactClusters && rv.hidden <= kSplitMaxCols && rv.hidden % 128u == 0u;
   float scale = 1.0f;
   bool have_scale = !rv.rms;
   bool full = false;
   float m = -INFINITY;
   for (;;) {
     // Candidates: a compact list in out.cl, wavefront by wavefront.
-    bool member[PER];
+    bool member[PER], above = false;
     uint32_t mine = 0;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const uint32_t e = base + j;
+      const float hi = l[j] + kBoundSlack * b[j];
       // A bound that is not finite admits the expert (NaN comparisons fail).
-      member[j] = e < E && (full || !(l[j] + kBoundSlack * b[j] + tie_margin(mx, l[j]) < th));
+      member[j] = e < E && (full || !(hi + tie_margin(top, l[j]) < th));
+      above |= e < E && hi > top + 1.0f;
       mine += member[j] ? 1u : 0u;
     }
     const float incl = wave_incl_scan(static_cast<float>(mine));  // small integers: exact
-    if (lane == kWave - 1) out.wcount[wave] = static_cast<uint32_t>(incl);
+    const uint32_t flag = __any(above) ? 1u << 16 : 0u;
+    if (lane == kWave - 1) out.wcount[wave] = static_cast<uint32_t>(incl) | flag;
     __syncthreads();
     uint32_t pos = static_cast<uint32_t>(incl) - mine;
-    for (uint32_t w = 0; w < wave; ++w) pos += out.wcount[w];
-    const uint32_t nc = out.wcount[0] + out.wcount[1] + out.wcount[2] + out.wcount[3];
+    for (uint32_t w = 0; w < wave; ++w) pos += out.wcount[w] & 0xFFFFu;
+    uint32_t nc = (out.wcount[0] + out.wcount[1]) + (out.wcount[2] + out.wcount[3]);
+    // An expert outside the picks whose logit might be the largest by more than
+    // the tie margin allows for: the list may lack a probability equal to a pick's.
+    if (nc > 0xFFFFu && !full) {
+      if (tid == 0) out.nneartie = 0u;
+      full = true;
+      __syncthreads();
+      continue;
+    }
+    nc &= 0xFFFFu;
     uint32_t cpos[PER];  // list position of each member
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
@@ -1169,7 +1191,7 @@ __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[P
     if constexpr (MODE == kExactClusters) {
       if (clusters && !full && nc <= kWave) {
         clusters = false;
-        if (resolve_clusters(rv, t, out, mx, nc)) {
+        if (resolve_clusters(rv, t, out, nc)) {
           if (tid == 0) {
             out.nneartie = 0u;
             out.ncand = nc;
@@ -1499,8 +1521,9 @@ __device__ __forceinline__ void select_values(const RouteView& rv, uint32_t t, c
 
   // The certificate: every expert outside the picks below the k-th's lower
   // bound, each adjacent pair of picks far enough apart (one thread per
-  // pair), and the k-th pick far from underflow.
-  const float lk = out.lg[k - 1];
+  // pair), and the k-th pick far from underflow. Where the order is proven the
+  // first pick's upper bound is the largest.
+  const float lk = out.lg[k - 1], top = mx + kBoundSlack * out.bd[0];
   const float low = lk - kBoundSlack * out.bd[k - 1];
   const uint64_t kth = (static_cast<uint64_t>(ordered_key(lk)) << 32) | ~out.id[k - 1];
   bool bad = false;
@@ -1508,20 +1531,20 @@ __device__ __forceinline__ void select_values(const RouteView& rv, uint32_t t, c
   for (int j = 0; j < PER; ++j) {
     const uint32_t e = base + j;
     const uint64_t c = (static_cast<uint64_t>(ordered_key(l[j])) << 32) | ~e;
-    if (e < E && c < kth && !(l[j] + kBoundSlack * b[j] + tie_margin(mx, l[j]) < low)) bad = true;
+    if (e < E && c < kth && !(l[j] + kBoundSlack * b[j] + tie_margin(top, l[j]) < low)) bad = true;
   }
   if (tid + 1u < k) {
     const uint32_t i = tid;
     const float need = kBoundSlack * (out.bd[i] + out.bd[i + 1]) +
-                       (out.id[i] > out.id[i + 1] ? tie_margin(mx, out.lg[i + 1]) : 0.0f);
+                       (out.id[i] > out.id[i + 1] ? tie_margin(top, out.lg[i + 1]) : 0.0f);
     if (!(out.lg[i] - out.lg[i + 1] > need)) bad = true;
   }
-  if (tid == 0 && !(lk - mx >= -kUnderflowGap)) bad = true;
+  if (tid == 0 && !(low - top >= -kUnderflowGap)) bad = true;
   bad = __syncthreads_or(bad) != 0;
   OSMD_STAMP(7, timeline_first());
   if (need_p) sum = ((out.red[2][0] + out.red[2][1]) + out.red[2][2]) + out.red[2][3];
   bool full = false;
-  if (bad) full = select_exact<PER, MODE>(rv, t, l, b, out, mx);
+  if (bad) full = select_exact<PER, MODE>(rv, t, l, b, out);
   if (need_p && tid < k) out.p[tid] = expf(out.lg[tid] - mx) / sum;
   if (tid == 0) out.flags = (bad ? 1u : 0u) | (full ? 2u : 0u);
   if (count && tid == 0 && rv.stats != nullptr) {

@@ -68,28 +68,22 @@ def rows_for(logits):
     return router
 
 
-def every_selection(ctx, router, k, x=None, sublayers=(False, True)):
-    """(label, ids, stats) of each kernel that selects: one token and four (inside gate/up), 16 (the selection kernel
+def every_selection(ctx, router, k, x, xin, nw):
+    """(label, ids, stats) of each kernel that selects for the router's input x (xin, normalised with nw): one token and four (inside gate/up), 16 (the selection kernel
     behind the per-token router), 48 (behind the router GEMM), with and without the norm, and 1,024 bf16 tokens."""
     E, D = router.shape
     I, G = 128, 64
     g = osm_hip.geometry(D, I, G, osm_hip.BF16)
     slab = osm_hip.ExpertSlab(ctx, g, 1, E)
     slab.synthesize(1)
-    nw = np.full(D, 1 / 16, np.float32)
     moe = osm_hip.MoeLayer(ctx, g, E, k, router, osm_hip.F32, None, nw, None, max_tokens=1024, rms_eps=1e-20)
-    if x is None:
-        x = np.zeros(D, np.float32)
-        x[0] = 1.0
-    for sublayer in sublayers:
-        xin = 16 * x if sublayer else x
-        if sublayer:
-            assert np.array_equal(O.rms_norm(xin, 1, D, nw, 1e-20), x)
+    assert np.array_equal(O.rms_norm(xin, 1, D, nw, 1e-20), x)
+    for sublayer in (False, True):
         for T, path in ((1, osm_hip.PATH_PER_TOKEN), (4, osm_hip.PATH_PER_TOKEN), (16, osm_hip.PATH_PER_TOKEN),
                         (48, osm_hip.PATH_GROUPED)):
             moe.set_path(path)
             xd, yd = ctx.alloc(T * D * 4), ctx.alloc(T * D * 4)
-            xd.upload(np.tile(xin, (T, 1)))
+            xd.upload(np.tile(xin if sublayer else x, (T, 1)))
             moe.routing_stats(reset=True)
             moe.decode_device(slab, 0, xd.ptr, yd.ptr, T, sublayer=sublayer)
             yield (T, sublayer), moe.routing(T)["ids"], moe.routing_stats()
@@ -102,11 +96,14 @@ def every_selection(ctx, router, k, x=None, sublayers=(False, True)):
 
 
 def check_every_selection(ctx, logits, k):
-    router = rows_for(logits)
     x = np.zeros(EXACT_D, np.float32)
     x[0] = 1.0
-    want = O.route_qwen_top_k(x, router, EXACT_D, len(logits), k, True)["ids"]
-    for label, ids, _ in every_selection(ctx, router, k):
+    return check_rows(ctx, rows_for(logits), k, x, 16 * x, 1 / 16)
+
+
+def check_rows(ctx, router, k, x, xin, nw):
+    want = O.route_qwen_top_k(x, router, EXACT_D, len(router), k, True)["ids"]
+    for label, ids, _ in every_selection(ctx, router, k, x, xin, np.full(EXACT_D, nw, np.float32)):
         assert np.array_equal(ids, np.tile(want, (len(ids), 1))), (label, ids[0], want)
     return list(want)
 
@@ -153,3 +150,34 @@ def quotient_tie(extra):
 @pytest.mark.parametrize("extra", [0, 70])
 def test_quotient_tie_behind_an_equal_exp(ctx, extra):
     assert check_every_selection(ctx, quotient_tie(extra), 2) == [0, 10]
+
+
+# Logits that the reference's fp32 sums move by tens (inputs of 1; a little over 2^26, then n columns of +-4, half a
+# unit in its last place, which they drop, then the first taken off again; the rest in the last column). What the device's fp64 sums say of the distance to
+# the largest logit is then no guide to the reference's exps.
+def moved(row, n, step, ref):
+    big = 2.0**26 + 16
+    row[0], row[1:n + 1], row[n + 1], row[-1] = big, step, -big, ref
+
+
+def distance_rows(case):
+    router = np.zeros((40, EXACT_D), np.float32)
+    router[:, -1] = -2000
+    if case == "open":  # 100 and, by the device's sums, 30 and 28: for the reference 150 and more below, p = 0
+        router[0, -1] = 100
+        moved(router[33], 20, 4, -50)
+        moved(router[36], 22, 4, -60)
+    elif case == "proven":  # 0 and -79, apart by their bounds: for the reference -127, p = 0
+        router[0, -1] = 0
+        moved(router[36], 12, 4, -127)
+    else:  # -1 for the device, 59 for the reference, 58.5 above three logits that round to one distance from it
+        moved(router[5], 15, -4, 59)
+        router[20, -1] = router[30, -1] = 0.5
+        router[10, -1] = 0.5 - 13 * 2.0**-23
+    return router
+
+
+@pytest.mark.parametrize("case,want", [("open", [0, 1]), ("proven", [0, 1]), ("above", [5, 10])])
+def test_distance_from_the_largest_logit(ctx, case, want):
+    x = np.ones(EXACT_D, np.float32)
+    assert check_rows(ctx, distance_rows(case), 2, x, x, 1.0) == want
