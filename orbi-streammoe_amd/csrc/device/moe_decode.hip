@@ -92,7 +92,7 @@ struct RouteView {
   const float* logits;                // [B, E]
   const float* bounds;                // [B, E] bound of each logit, or null (no bound: exact path)
   const float* planes;                // null, or `parts` planes [B][E + 1] of partial sums
-  const float* planes_lo;             // with planes: what their rounding to fp32 left, or null
+  const double* planes64;             // or the planes in fp64 (a router that is not bf16)
   const float* bound_planes;          // with planes: [parts][B][E + 1] bound parts, or null
   uint32_t parts, tokens;
   float* logits_out;                  // [B, E]  with planes: the summed logits
@@ -1584,45 +1584,45 @@ __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Se
   const uint32_t D = rv.hidden;
   const float* lg = rv.logits + static_cast<size_t>(t) * E;
   const uint32_t base = threadIdx.x * PER;
+  const bool planes = PLANES && (rv.planes != nullptr || rv.planes64 != nullptr);
   float p[PER], bnd[PER];
   const uint8_t* tab[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const uint32_t e = (base + j < E) ? base + j : E - 1u;  // clamped: every load in bounds
-    if (PLANES && rv.planes != nullptr) {
+    if (planes) {
       // Partial sums of the router GEMM's K ranges, added in plane order.
       // Range r of R columns starts at the running sum P_r, so its prefix
       // sums are bounded by R |P_r| plus the plane's own part.
       const size_t ps = static_cast<size_t>(rv.tokens) * (E + 1u);
       const size_t o = static_cast<size_t>(t) * (E + 1u) + e;
-      const float* pl = rv.planes + o;
       const bool bounded = rv.bound_planes != nullptr;
       const float cols = static_cast<float>(D / rv.parts);
       float v, rs = 0.0f;
-      if (rv.planes_lo != nullptr) {
-        // Planes of fp64 sums: added up in fp64, rounded once.
-        const float* plo = rv.planes_lo + o;
+      if (rv.planes64 != nullptr) {
+        // Added up in fp64, rounded once.
         double vd = 0.0;
         for (uint32_t p0 = 0; p0 < rv.parts; p0 += 4u) {
-          float hi[4], lo[4], rb[4];
+          double pd[4];
+          float rb[4];
 #pragma unroll
           for (uint32_t i = 0; i < 4u; ++i) {
             const uint32_t part = p0 + i < rv.parts ? p0 + i : p0;  // read again, not added
-            hi[i] = pl[part * ps];
-            lo[i] = plo[part * ps];
+            pd[i] = rv.planes64[part * ps + o];
             rb[i] = bounded ? rv.bound_planes[part * ps + o] : 0.0f;
           }
 #pragma unroll
           for (uint32_t i = 0; i < 4u; ++i) {
             if (p0 + i < rv.parts) {
               rs += rb[i] + cols * fabsf(static_cast<float>(vd));
-              vd += static_cast<double>(hi[i]) + lo[i];
+              vd += pd[i];
             }
           }
         }
         v = static_cast<float>(vd);
       } else if (rv.parts <= kMaxPlanes) {
         // Every plane's loads issued before the first addition.
+        const float* pl = rv.planes + o;
         float pv[kMaxPlanes], rb[kMaxPlanes];
 #pragma unroll
         for (uint32_t part = 0; part < kMaxPlanes; ++part) {
@@ -1641,6 +1641,7 @@ __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Se
           }
         }
       } else {
+        const float* pl = rv.planes + o;
         v = pl[0];
         if (bounded) rs = rv.bound_planes[o];
         for (uint32_t part = 1; part < rv.parts; ++part) {
@@ -1659,16 +1660,16 @@ __device__ __forceinline__ void select_block(const RouteView& rv, uint32_t t, Se
     }
     tab[j] = rv.expert_table ? rv.expert_table[e] : nullptr;
   }
-  if (PLANES && rv.planes != nullptr && rv.has_shared && threadIdx.x == 0) {
+  if (planes && rv.has_shared && threadIdx.x == 0) {
     const size_t ps = static_cast<size_t>(rv.tokens) * (E + 1u);
     const size_t o = static_cast<size_t>(t) * (E + 1u) + E;
-    float g = rv.planes[o];
-    if (rv.planes_lo != nullptr) {
+    float g;
+    if (rv.planes64 != nullptr) {
       double gd = 0.0;
-      for (uint32_t part = 0; part < rv.parts; ++part)
-        gd += static_cast<double>(rv.planes[o + part * ps]) + rv.planes_lo[o + part * ps];
+      for (uint32_t part = 0; part < rv.parts; ++part) gd += rv.planes64[o + part * ps];
       g = static_cast<float>(gd);
     } else {
+      g = rv.planes[o];
       for (uint32_t part = 1; part < rv.parts; ++part) g += rv.planes[o + part * ps];
     }
     rv.gate_out[t] = 1.0f / (1.0f + expf(-g));  // reference_ops.cpp:214-216
@@ -2261,7 +2262,7 @@ __global__ __launch_bounds__(kDownThreads) void down_kernel(DownParams p) {
 // matrix cores, v_mfma_f64_16x16x4. As one wavefront per token and router row
 // the 8-bit router of a 512-token pass took 400 µs, more than twice the
 // experts' gate and up GEMM; this takes 48 µs, with the same products (exact
-// in fp64) and the logit rounded once: the same bits. (Three bf16 terms per
+// in fp64), summed in fp64 to the end and rounded once. (Three bf16 terms per
 // element on the bf16 cores took 51 µs and came out with 2.8 times the
 // logits' error.)
 //
@@ -2377,9 +2378,9 @@ __device__ __forceinline__ float raw64_get(const Raw64<RD>& r, int j, int i) {
 template <int RD, int NB, bool XBF16>
 __global__ __launch_bounds__(256) void router_f64_kernel(
     const void* __restrict__ x, uint32_t T, uint32_t D, const void* __restrict__ router,
-    const void* __restrict__ shared_gate_vec, uint32_t E, uint32_t group, uint32_t rms, float* __restrict__ planes,
-    float* __restrict__ planes_lo, const float* __restrict__ rnorm, const float* __restrict__ xnorm,
-    float* __restrict__ bplanes, uint32_t gx, uint32_t gy, uint32_t gz) {
+    const void* __restrict__ shared_gate_vec, uint32_t E, uint32_t group, uint32_t rms, double* __restrict__ planes,
+    const float* __restrict__ rnorm, const float* __restrict__ xnorm, float* __restrict__ bplanes, uint32_t gx,
+    uint32_t gy, uint32_t gz) {
   typedef double f64x4 __attribute__((ext_vector_type(4)));
   constexpr uint32_t R = 16u * NB;
   constexpr uint32_t RS = R + 4u;  // LDS row stride (floats), padded against bank conflicts
@@ -2470,10 +2471,8 @@ __global__ __launch_bounds__(256) void router_f64_kernel(
       ap = fmaf(rn[c].w, xv.w, ap);
     }
     const size_t o = (static_cast<size_t>(bz) * T + t) * (E + 1u) + row;
-    const float hi = static_cast<float>(acc[v]);
-    planes[o] = hi;
-    planes_lo[o] = static_cast<float>(acc[v] - hi);
-    bplanes[o] = 16.0f * static_cast<float>(sabs[v]) + fabsf(hi) + ca * ap;
+    planes[o] = acc[v];
+    bplanes[o] = 16.0f * static_cast<float>(sabs[v]) + fabsf(static_cast<float>(acc[v])) + ca * ap;
   }
 }
 
@@ -2622,8 +2621,7 @@ int launch_route_rd(const osmd_moe_args& a, hipStream_t st) {
 
 template <int RD, int NB>
 int launch_router_f64_range(const osmd_moe_args& a, const void* x, uint32_t x_bf16, const float* router_norms,
-                            const float* x_norms, float* planes, float* planes_lo, float* bound_planes,
-                            hipStream_t st) {
+                            const float* x_norms, double* planes, float* bound_planes, hipStream_t st) {
   const uint32_t T = a.tokens, D = a.geom.hidden, E = a.expert_count;
   const bool shared = (a.flags & OSMD_MOE_SHARED) != 0u;
   const uint32_t gx = (E + (shared ? 1u : 0u) + 63u) / 64u, gz = D / (16u * NB);
@@ -2631,7 +2629,7 @@ int launch_router_f64_range(const osmd_moe_args& a, const void* x, uint32_t x_bf
   const uint32_t launch = (gx * gy * gz + 7u) / 8u * 8u;
   auto go = [&](auto kernel) {
     kernel<<<launch, 256, 0, st>>>(x, T, D, a.router, shared ? a.shared_gate_vec : nullptr, E, a.router_group,
-                                   (a.flags & OSMD_MOE_RMSNORM) ? 1u : 0u, planes, planes_lo, router_norms, x_norms,
+                                   (a.flags & OSMD_MOE_RMSNORM) ? 1u : 0u, planes, router_norms, x_norms,
                                    bound_planes, gx, gy, gz);
   };
   x_bf16 ? go(router_f64_kernel<RD, NB, true>) : go(router_f64_kernel<RD, NB, false>);
@@ -2640,15 +2638,15 @@ int launch_router_f64_range(const osmd_moe_args& a, const void* x, uint32_t x_bf
 
 template <int RD>
 int launch_router_f64(const osmd_moe_args& a, const void* x, uint32_t x_bf16, uint32_t cols, const float* router_norms,
-                      const float* x_norms, float* planes, float* planes_lo, float* bound_planes, hipStream_t st) {
+                      const float* x_norms, double* planes, float* bound_planes, hipStream_t st) {
   if (cols == 0u || a.geom.hidden % cols != 0u) return static_cast<int>(hipErrorInvalidValue);
   switch (cols) {
     case 512:
-      return launch_router_f64_range<RD, 32>(a, x, x_bf16, router_norms, x_norms, planes, planes_lo, bound_planes, st);
+      return launch_router_f64_range<RD, 32>(a, x, x_bf16, router_norms, x_norms, planes, bound_planes, st);
     case 256:
-      return launch_router_f64_range<RD, 16>(a, x, x_bf16, router_norms, x_norms, planes, planes_lo, bound_planes, st);
+      return launch_router_f64_range<RD, 16>(a, x, x_bf16, router_norms, x_norms, planes, bound_planes, st);
     case 128:
-      return launch_router_f64_range<RD, 8>(a, x, x_bf16, router_norms, x_norms, planes, planes_lo, bound_planes, st);
+      return launch_router_f64_range<RD, 8>(a, x, x_bf16, router_norms, x_norms, planes, bound_planes, st);
     default: return static_cast<int>(hipErrorInvalidValue);
   }
 }
@@ -2657,7 +2655,7 @@ RouteView route_view(const osmd_moe_args& a) {
   RouteView rv;
   rv.logits = a.logits;
   rv.planes = a.logit_planes;
-  rv.planes_lo = a.logit_planes_lo;
+  rv.planes64 = a.logit_planes64;
   rv.parts = a.logit_parts;
   rv.tokens = a.tokens;
   rv.logits_out = a.logits;
@@ -2771,18 +2769,18 @@ int osmd_router_norms(const osmd_moe_args* a, float* norms, osmd_stream s) {
 }
 
 int osmd_router_f64(const osmd_moe_args* a, const void* x, uint32_t x_bf16, uint32_t parts, const float* router_norms,
-                    const float* x_norms, float* planes, float* planes_lo, float* bound_planes, osmd_stream s) {
+                    const float* x_norms, double* planes, float* bound_planes, osmd_stream s) {
   const uint32_t cols = parts != 0u ? a->geom.hidden / parts : 0u;
   switch (a->router_dtype) {
     case OSM_META_F32:
-      return launch_router_f64<OSM_META_F32>(*a, x, x_bf16, cols, router_norms, x_norms, planes, planes_lo,
-                                             bound_planes, static_cast<hipStream_t>(s));
+      return launch_router_f64<OSM_META_F32>(*a, x, x_bf16, cols, router_norms, x_norms, planes, bound_planes,
+                                             static_cast<hipStream_t>(s));
     case OSM_META_F16:
-      return launch_router_f64<OSM_META_F16>(*a, x, x_bf16, cols, router_norms, x_norms, planes, planes_lo,
-                                             bound_planes, static_cast<hipStream_t>(s));
+      return launch_router_f64<OSM_META_F16>(*a, x, x_bf16, cols, router_norms, x_norms, planes, bound_planes,
+                                             static_cast<hipStream_t>(s));
     case OSM_ROUTER_AFFINE_Q8:
-      return launch_router_f64<OSM_ROUTER_AFFINE_Q8>(*a, x, x_bf16, cols, router_norms, x_norms, planes, planes_lo,
-                                                     bound_planes, static_cast<hipStream_t>(s));
+      return launch_router_f64<OSM_ROUTER_AFFINE_Q8>(*a, x, x_bf16, cols, router_norms, x_norms, planes, bound_planes,
+                                                     static_cast<hipStream_t>(s));
     default: return static_cast<int>(hipErrorInvalidValue);
   }
 }
@@ -2800,7 +2798,7 @@ int osmd_moe_gate_up(const osmd_moe_args* a, osmd_stream s) {
   const int per = a->expert_table ? selection_per(a->expert_count) : 0;
   // gate/up's own selection reads final logits (the per-token router's);
   // router GEMM planes go through the select kernel.
-  if (per > 0 && a->logit_planes != nullptr) return static_cast<int>(hipErrorInvalidValue);
+  if (per > 0 && (a->logit_planes != nullptr || a->logit_planes64 != nullptr)) return static_cast<int>(hipErrorInvalidValue);
   return launch_gate_up(gate_up_params(*a), a->tokens, per, static_cast<hipStream_t>(s));
 }
 

@@ -1552,7 +1552,7 @@ int osmd_moe_grouped(const osmd_moe_grouped_args* a, osmd_stream s) {
   // path's 40 tokens on, reading x itself (one 512-token pass of an 8-bit
   // router: 400 µs as per-token GEMVs, 48 µs).
   const bool router_f64 = m.router_dtype != OSM_META_BF16 && T >= OSMD_GROUPED_MIN_TOKENS &&
-                          a->logit_planes_lo != nullptr && a->router_norms != nullptr && a->x_norms != nullptr &&
+                          a->logit_planes64 != nullptr && a->router_norms != nullptr && a->x_norms != nullptr &&
                           a->bound_planes != nullptr;
   if (xbf16 && !router_gemm && !router_f64) {
     // The per-token kernel takes fp32 input.
@@ -1616,11 +1616,10 @@ int osmd_moe_grouped(const osmd_moe_grouped_args* a, osmd_stream s) {
     ms.bound_planes = gemm_bounds ? a->bound_planes : nullptr;
   } else if (router_f64) {
     ms.logit_parts = D / router_range(D);
-    r = osmd_router_f64(&m, xin, xbf16 ? 1u : 0u, ms.logit_parts, a->router_norms, xnorms, a->logit_planes,
-                        a->logit_planes_lo, a->bound_planes, s);
+    r = osmd_router_f64(&m, xin, xbf16 ? 1u : 0u, ms.logit_parts, a->router_norms, xnorms, a->logit_planes64,
+                        a->bound_planes, s);
     if (r != 0) return r;
-    ms.logit_planes = a->logit_planes;
-    ms.logit_planes_lo = a->logit_planes_lo;
+    ms.logit_planes64 = a->logit_planes64;
     ms.bound_planes = a->bound_planes;
   } else {
     // The decode router kernel, one token per grid row (fp32 input).

@@ -153,9 +153,10 @@ typedef struct osmd_moe_args {
   /* Router partial sums (the grouped router GEMM splits K): when logit_planes
    * is set, it holds logit_parts planes [B][E + 1] (column E: the shared-gate
    * dot) that the selection adds in plane order, writing logits and
-   * shared_gate itself; when null, logits and shared_gate are final. */
+   * shared_gate itself; logit_planes64 is the same in fp64 (the sums are then
+   * rounded once). With both null, logits and shared_gate are final. */
   const float* logit_planes;
-  const float* logit_planes_lo; /* what the planes' rounding to fp32 left, or null */
+  const double* logit_planes64;
   uint32_t logit_parts;
   /* Routing exactness. logit_bounds [B, E]: the router writes, for every
    * logit, a bound on its distance from the reference's sequentially summed
@@ -235,7 +236,7 @@ int osmd_moe_combine(const osmd_moe_args* a, const float* parts, osmd_stream s);
  *   gu_part  f32 [splits(D)][2][P][I]
  *   h_terms  bf16 [P][2][I]    h_sums   f32 [P][I/G]
  *   partial  f32 [splits(I)][P][D]
- *   logit_planes f32 [osmd_moe_grouped_router_parts(D)][T][E + 1] (router GEMM partials)
+ *   logit_planes f32 (or logit_planes64 f64) [osmd_moe_grouped_router_parts(D)][T][E + 1] (router GEMM partials)
  * where splits(n) = osmd_moe_grouped_splits(&moe.geom, n) K ranges of the
  * n columns (hidden for gate/up, inter for down).
  * plus the decode workspace of moe (logits, ids, weights, mass, shared_gate,
@@ -261,10 +262,9 @@ typedef struct osmd_moe_grouped_args {
   const float* router_norms;
   float* x_norms;
   float* bound_planes;
-  /* Low parts of the logit planes of a router that is not bf16, the shape of
-   * logit_planes, or null: such a router then runs as one GEMV per token and
-   * row. */
-  float* logit_planes_lo;
+  /* The logit planes of a router that is not bf16, in fp64, or null: such a
+   * router then runs as one GEMV per token and row. */
+  double* logit_planes64;
 } osmd_moe_grouped_args;
 /* Tokens from which a layer's decodes take the grouped path by themselves,
  * and from which a router that is not bf16 runs as a GEMM. */
@@ -275,9 +275,9 @@ int osmd_router_norms(const osmd_moe_args* a, float* norms, osmd_stream s);
 /* The router of a->tokens tokens as a GEMM in fp64, any dtype but bf16: x
  * [T, D] (fp32, or bf16 when x_bf16; already normalised) against a->router
  * and the shared gate, in `parts` = D / 512, 256 or 128 K ranges whose fp64
- * sums go to planes + planes_lo, with the bound planes the selection reads. */
+ * sums go to planes, with the bound planes the selection reads. */
 int osmd_router_f64(const osmd_moe_args* a, const void* x, uint32_t x_bf16, uint32_t parts, const float* router_norms,
-                    const float* x_norms, float* planes, float* planes_lo, float* bound_planes, osmd_stream s);
+                    const float* x_norms, double* planes, float* bound_planes, osmd_stream s);
 size_t osmd_moe_grouped_max_tiles(uint32_t tokens, uint32_t nslot, uint32_t experts);
 uint32_t osmd_moe_grouped_splits(const osm_expert_geometry* g, uint32_t cols);
 uint32_t osmd_moe_grouped_router_parts(uint32_t hidden);

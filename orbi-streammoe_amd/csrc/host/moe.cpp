@@ -154,7 +154,7 @@ struct HipMoeLayer::Impl {
   // workspace (every layer on one stream uses the same memory in turn)
   HipMoePath path = HipMoePath::automatic;
   enum GroupedBuf { kXTerms, kXSums, kPairPos, kPairW, kTiles, kTileCount, kGuPart, kHTerms, kHSums, kPartial,
-                    kLogitPlanes, kXNorms, kBoundPlanes, kLogitPlanesLo, kGroupedBufs };
+                    kLogitPlanes, kXNorms, kBoundPlanes, kGroupedBufs };
   std::array<std::size_t, kGroupedBufs> g_off{};
   std::size_t g_bytes = 0;
   std::uint8_t* g_base = nullptr;
@@ -173,10 +173,9 @@ struct HipMoeLayer::Impl {
         osmd_moe_grouped_splits(&g, static_cast<std::uint32_t>(D)) * 2U * P * I * 4U,  // gate/up partials
         P * 2U * I * 2U, P * (I / G) * 4U,                                          // h terms, h sums
         osmd_moe_grouped_splits(&g, static_cast<std::uint32_t>(I)) * P * D * 4U,   // down partials
-        parts * T * (cfg.expert_count + 1U) * 4U,                                   // logit planes
+        parts * T * (cfg.expert_count + 1U) * (router_f64() ? 8U : 4U),             // logit planes
         T * (D / 32U) * 4U,                                                         // input chunk norms
-        parts * T * (cfg.expert_count + 1U) * 4U,                                   // bound planes
-        router_f64() ? parts * T * (cfg.expert_count + 1U) * 4U : 0U};              // low parts of the logit planes
+        parts * T * (cfg.expert_count + 1U) * 4U};                                  // bound planes
     std::size_t off = 0;
     for (std::size_t i = 0; i < bytes.size(); ++i) {
       g_off[i] = off;
@@ -225,11 +224,13 @@ struct HipMoeLayer::Impl {
     ga.h_terms = gbuf<std::uint16_t>(kHTerms);
     ga.h_sums = gbuf<float>(kHSums);
     ga.partial = gbuf<float>(kPartial);
-    ga.logit_planes = gbuf<float>(kLogitPlanes);
+    if (router_f64())
+      ga.logit_planes64 = gbuf<double>(kLogitPlanes);
+    else
+      ga.logit_planes = gbuf<float>(kLogitPlanes);
     ga.router_norms = router_norms.as<const float>();
     ga.x_norms = gbuf<float>(kXNorms);
     ga.bound_planes = gbuf<float>(kBoundPlanes);
-    ga.logit_planes_lo = router_f64() ? gbuf<float>(kLogitPlanesLo) : nullptr;
     return ga;
   }
 

@@ -2,6 +2,8 @@
 picks against the oracle's, at the K ranges, token tiles and router rows
 where the GEMM's edges lie."""
 
+import math
+
 import numpy as np
 import pytest
 
@@ -37,7 +39,7 @@ def layer(ctx, kind, D, E, k, T, seed):
 def check(moe, x, value, gate, E, k):
     r = moe.routing(len(x))
     exact = x.astype(np.float64) @ value.astype(np.float64).T
-    # Summed in fp64 and rounded to fp32 once, whatever of the planes' 48 bits is lost below that.
+    # Summed in fp64 (at most 2,048 roundings of 2^-53) and rounded to fp32 once.
     bound = 2.0**-24 * np.abs(exact) + 2.0**-40 * (np.abs(x).astype(np.float64) @ np.abs(value).astype(np.float64).T)
     assert np.all(np.abs(r["logits"] - exact) <= bound)
     for t in range(len(x)):
@@ -70,3 +72,27 @@ def test_router_f64(ctx, D, E, T, kind):
     xd.upload(bits)
     moe.prefill_device(slab, 0, xd.ptr, yd.ptr, T)
     check(moe, (bits.astype(np.uint32) << 16).view(np.float32).reshape(T, D), value, gate, E, k)
+
+
+def test_partial_sums_in_fp64(ctx):
+    # Five K ranges of 128 columns. Rows 0-31: 2^26 at the end of the first, taken off at the end of the second, the
+    # rest multiples of 2^-24 below 1. Their sums are exact in fp64, and the logit is the exact sum rounded once; ranges
+    # held in 48 bits would be off by up to 2^-22. Row 32: the second range's own sum is beyond fp32, the running sums
+    # of the reference are not.
+    rng = np.random.default_rng(1)
+    D, E, k, T = 640, 64, 6, 40
+    w = (rng.integers(-2**24, 2**24, (E, D)) * 2.0**-24).astype(np.float32)
+    w[:32, 127], w[:32, 255] = 2.0**26, -(2.0**26)
+    w[32] = 0
+    w[32, [0, 128, 129, 256, 639]] = [-3e38, 3e38, 3e38, -3e38, 20]
+    g = osm_hip.geometry(D, 128, 64, osm_hip.BF16)
+    slab = osm_hip.ExpertSlab(ctx, g, 1, E)
+    slab.synthesize(1)
+    moe = osm_hip.MoeLayer(ctx, g, E, k, w, osm_hip.F32, None, None, None, max_tokens=T)
+    want = np.array([math.fsum(row) for row in w.tolist()], np.float32)
+    ids = O.route_qwen_top_k(np.ones(D, np.float32), w, D, E, k, True)["ids"]
+    for path in (osm_hip.PATH_PER_TOKEN, osm_hip.PATH_GROUPED):
+        moe.set_path(path)
+        r = moe.run_slab(slab, 0, np.ones((T, D), np.float32))
+        assert np.array_equal(r["logits"], np.tile(want, (T, 1))), path
+        assert np.array_equal(r["ids"], np.tile(ids, (T, 1))), path
