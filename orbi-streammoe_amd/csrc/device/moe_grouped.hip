@@ -146,10 +146,12 @@ __device__ __forceinline__ void prepare_word(const float (&v)[8], bool in, size_
     // Euclidean norm of each 32-column chunk (4 words), rounded up: the
     // router GEMM's error bounds take |w . x| <= |w| |x| per chunk. The
     // fp32 sum of 32 squares is within 32 u of the true one, so 1 + 2^-20
-    // covers it and the square root's rounding.
+    // covers it and the square root's rounding; 2^-72 covers squares rounded
+    // as subnormals or to zero (32 of them, 2^-150 each), and keeps the
+    // product with an infinite row norm from being NaN.
     sq += __shfl_xor(sq, 1, kWave);
     sq += __shfl_xor(sq, 2, kWave);
-    if (in && (i % 4u) == 0u) norms[i / 4u] = sqrtf(sq) * (1.0f + 0x1p-20f);
+    if (in && (i % 4u) == 0u) norms[i / 4u] = sqrtf(sq) * (1.0f + 0x1p-20f) + 0x1p-72f;
   }
 }
 

@@ -9,7 +9,7 @@ import pytest
 
 import oracle as O
 import osm_hip
-from helpers import max_abs
+from helpers import bf16_bits, bf16_to_f32, max_abs
 from test_gpu_router_q8 import dequant, quantize_q8
 
 pytestmark = pytest.mark.gpu
@@ -96,3 +96,30 @@ def test_partial_sums_in_fp64(ctx):
         r = moe.run_slab(slab, 0, np.ones((T, D), np.float32))
         assert np.array_equal(r["logits"], np.tile(want, (T, 1))), path
         assert np.array_equal(r["ids"], np.tile(ids, (T, 1))), path
+
+
+# Inputs whose squares are below fp32's smallest number, against a router large enough for logits of the usual size: the
+# bounds have to know the products' size all the same. Each expert's columns are blocks of 16, eight values and their
+# negatives in an order of its own, which leave nothing, and its logit in the last column; the reference's sums of them
+# are off by a multiple of the gaps between the logits, token by token.
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+def test_bounds_of_tiny_inputs(ctx, kind):
+    rng = np.random.default_rng(4)
+    D, E, k, T = 384, 64, 6, 48
+    a = np.abs(bf16_to_f32(bf16_bits(rng.normal(0, 1e4, (23, 8)))))
+    w = np.zeros((E, D), np.float32)
+    for e in range(E):
+        for b in range(23):
+            w[e, 16 * b:16 * b + 16] = rng.permutation(np.concatenate([a[b], -a[b]]))
+        w[e, D - 1] = 1 + (37 * e % E) * 2.0**-7
+    w *= np.float32(2.0**80)
+    x = np.repeat((rng.uniform(0.5, 2, (T, 1)) * 2.0**-80).astype(np.float32), D, 1)
+    g = osm_hip.geometry(D, 128, 64, osm_hip.BF16)
+    slab = osm_hip.ExpertSlab(ctx, g, 1, E)
+    slab.synthesize(1)
+    r, code = (bf16_bits(w), osm_hip.BF16) if kind == "bf16" else (w, osm_hip.F32)
+    moe = osm_hip.MoeLayer(ctx, g, E, k, r, code, None, None, None, max_tokens=T)
+    moe.set_path(osm_hip.PATH_GROUPED)
+    got = moe.run_slab(slab, 0, x)["ids"]
+    for t in range(T):
+        assert np.array_equal(got[t], O.route_qwen_top_k(x[t], w, D, E, k, True)["ids"]), t
