@@ -1121,10 +1121,13 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
 // was recomputed. out.nneartie gets the picks that sent it to the full
 // recompute (near ties with a lower id behind them).
 // How a kernel's selection takes the exact path: kExactPlain the general form
-// alone (gate/up of several tokens, whose selection every workgroup repeats and
-// which wants three wavefronts to a SIMD: the clusters' code takes 194
-// registers where the rest takes 168, and 4 tokens' sublayers took 4% longer
-// with it); kExactClusters open clusters first, and the full recompute by
+// alone (gate/up, whose selection every workgroup repeats and which wants three
+// wavefronts to a SIMD: 151 to 168 registers. With the clusters' code and
+// full_logits it takes 212 to 236, two wavefronts: 4 tokens' sublayers took 4%
+// longer; one token's took, hidden 2,048, top-10 and the shared expert, µs a
+// layer, plain / with clusters, 22.1 / 25.4 at intermediate 640, 23.6 / 26.8 at
+// 768, and 20.6 / 20.4 and 19.1 / 19.0 at 512 with 600 and 512 experts);
+// kExactClusters open clusters first, and the full recompute by
 // full_logits; kExactDeep the general form with its loads two steps ahead (253
 // registers: either of the other two beside it spills or halves the
 // occupancy). The selection kernel takes clusters in the sublayer form, where
@@ -2039,7 +2042,7 @@ __global__ __launch_bounds__(256) void gate_up_kernel(GateUpParams p) {
       // forms the probabilities.
       const bool publisher = blockIdx.x == 0 && j == 0;
       OSMD_STAMP(4, timeline_first());
-      select_block<PER, false, ROWS == kGuRowsOneToken ? kExactClusters : kExactPlain>(rv, t, sel, false, publisher);
+      select_block<PER, false, kExactPlain>(rv, t, sel, false, publisher);
       OSMD_STAMP(8, timeline_first());
       rows(pick_blob(rv, sel, j));
       OSMD_STAMP(10, timeline_first());
