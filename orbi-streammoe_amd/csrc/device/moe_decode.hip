@@ -1128,14 +1128,18 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
 // layer, plain / with clusters, 22.1 / 25.4 at intermediate 640, 23.6 / 26.8 at
 // 768, and 20.6 / 20.4 and 19.1 / 19.0 at 512 with 600 and 512 experts);
 // kExactClusters open clusters first, and the full recompute by
-// full_logits; kExactDeep the general form with its loads two steps ahead (253
-// registers: either of the other two beside it spills or halves the
-// occupancy). The selection kernel takes clusters in the sublayer form, where
-// they also split the RMS scale's chain (64 tokens: 35 -> 29 µs a launch), and
+// full_logits; kExactDeep the general form with its loads two steps ahead (246
+// to 255 registers: either of the other two beside it spills or halves the
+// occupancy). The selection kernel takes clusters in the sublayer form of
+// hidden sizes that the split chains take, where they also split the RMS
+// scale's chain (64 tokens: 35 -> 29 µs a launch), and
 // from 1,024 tokens on, where one launch in three or four holds a full recompute
 // (4,096 tokens, two layers: 2,699 -> 2,627 µs). Otherwise the deep form:
 // behind the router GEMM's wider bounds the slowest token of a 512-token launch
-// has four open experts or more, two passes and up (29 µs a launch against 25).
+// has four open experts or more, two passes and up (29 µs a launch against 25),
+// and other hidden sizes have nothing of the clusters (sublayers, bf16 router, µs
+// a layer with the plain form / deep: hidden 4,096 101.6 / 99.6 at 16 tokens and
+// 185.6 / 181.1 at 64, 8,192 245.6 / 240.1 and 343.7 / 332.7).
 enum ExactMode : int { kExactPlain = 0, kExactClusters = 1, kExactDeep = 2 };
 template <int PER, ExactMode MODE>
 __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[PER], const float (&b)[PER],
@@ -1711,9 +1715,11 @@ __device__ __forceinline__ void publish_selection(const RouteView& rv, uint32_t 
   if (tid == 0) rv.mass[t] = mass;
 }
 
-template <int PER, ExactMode MODE>
-__global__ __launch_bounds__(kSelThreads) void select_kernel(RouteView rv) {
-  if constexpr (MODE == kExactDeep) rv.rms = 0u;  // launched without it alone: nothing of the norm is compiled in
+// NORM: compiled with the norm, for launches of the sublayer form and those
+// that may be of either.
+template <int PER, ExactMode MODE, bool NORM>
+__global__ __launch_bounds__(kSelThreads, 2) void select_kernel(RouteView rv) {
+  if constexpr (!NORM) rv.rms = 0u;
   __shared__ Selection<PER> sel;
   select_block<PER, true, MODE>(rv, blockIdx.x, sel, true);
   publish_selection(rv, blockIdx.x, threadIdx.x, sel);
@@ -2691,21 +2697,23 @@ RouteView route_view(const osmd_moe_args& a) {
 
 int launch_select(const osmd_moe_args& a, hipStream_t st) {
   const RouteView rv = route_view(a);
-  const bool clusters = rv.rms != 0u || a.tokens >= 1024u;  // ExactMode
-  switch (selection_per(a.expert_count)) {
-    case 2:
-      if (clusters)
-        select_kernel<2, kExactClusters><<<a.tokens, kSelThreads, 0, st>>>(rv);
-      else
-        select_kernel<2, kExactDeep><<<a.tokens, kSelThreads, 0, st>>>(rv);
-      break;
-    default:
-      if (clusters)
-        select_kernel<4, kExactClusters><<<a.tokens, kSelThreads, 0, st>>>(rv);
-      else
-        select_kernel<4, kExactDeep><<<a.tokens, kSelThreads, 0, st>>>(rv);
-      break;
-  }
+  // ExactMode. In the sublayer form the clusters need rows that the split
+  // chains take; others, up to 1,024 tokens, run the deep form.
+  const bool rms = rv.rms != 0u;
+  const bool clusters = a.tokens >= 1024u || (rms && rv.hidden <= kSplitMaxCols && rv.hidden % 128u == 0u);
+  auto go = [&](auto per) {
+    constexpr int kPer = decltype(per)::value;
+    if (clusters)
+      select_kernel<kPer, kExactClusters, true><<<a.tokens, kSelThreads, 0, st>>>(rv);
+    else if (rms)
+      select_kernel<kPer, kExactDeep, true><<<a.tokens, kSelThreads, 0, st>>>(rv);
+    else
+      select_kernel<kPer, kExactDeep, false><<<a.tokens, kSelThreads, 0, st>>>(rv);
+  };
+  if (selection_per(a.expert_count) == 2)
+    go(std::integral_constant<int, 2>{});
+  else
+    go(std::integral_constant<int, 4>{});
   return launch_status();
 }
 
