@@ -1116,10 +1116,6 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
   return out.nopen != ~0u;
 }
 
-// The exact path (every thread of the workgroup; out.id/lg/bd hold the
-// device ranking). Rewrites out.id and out.lg; returns whether every expert
-// was recomputed. out.nneartie gets the picks that sent it to the full
-// recompute (near ties with a lower id behind them).
 // How a kernel's selection takes the exact path: kExactPlain the general form
 // alone (gate/up, whose selection every workgroup repeats and which wants three
 // wavefronts to a SIMD: 151 to 168 registers. With the clusters' code and
@@ -1133,14 +1129,25 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
 // occupancy). The selection kernel takes clusters in the sublayer form of
 // hidden sizes that the split chains take, where they also split the RMS
 // scale's chain (64 tokens: 35 -> 29 µs a launch), and
-// from 1,024 tokens on, where one launch in three or four holds a full recompute
-// (4,096 tokens, two layers: 2,699 -> 2,627 µs). Otherwise the deep form:
-// behind the router GEMM's wider bounds the slowest token of a 512-token launch
+// from 1,024 tokens on for the full recompute's sake. One selection in some
+// 50,000 needs it (2 of 98,304 at hidden 2,048 with random inputs, none of as
+// many at 4,096), and in the deep form the whole launch waits 0.3 to 0.5 ms for
+// it (512 experts, bf16 router, no norm, µs a layer, deep / clusters: 4,096
+// tokens at hidden 2,048 1,041 / 779, 1,536 at 4,096 1,118 / 667). Launches
+// without one lose up to 1%: 1,024 tokens 213 / 215 at 2,048 and 364 / 368 at
+// 4,096, 4,096 tokens 663 / 660 and 1,230 / 1,244. At the 2% of 1,024-token
+// launches that have one, the two come to about the same. Otherwise the deep
+// form: behind the router GEMM's wider bounds the slowest token of a 512-token launch
 // has four open experts or more, two passes and up (29 µs a launch against 25),
 // and other hidden sizes have nothing of the clusters (sublayers, bf16 router, µs
 // a layer with the plain form / deep: hidden 4,096 101.6 / 99.6 at 16 tokens and
 // 185.6 / 181.1 at 64, 8,192 245.6 / 240.1 and 343.7 / 332.7).
 enum ExactMode : int { kExactPlain = 0, kExactClusters = 1, kExactDeep = 2 };
+
+// The exact path (every thread of the workgroup; out.id/lg/bd hold the
+// device ranking). Rewrites out.id and out.lg; returns whether every expert
+// was recomputed. out.nneartie gets the picks that sent it to the full
+// recompute (near ties with a lower id behind them).
 template <int PER, ExactMode MODE>
 __device__ bool select_exact(const RouteView& rv, uint32_t t, const float (&l)[PER], const float (&b)[PER],
                              Selection<PER>& out) {
