@@ -71,10 +71,11 @@ def test_q8_router_decode_matches_fp32_and_oracle(ctx, group):
         assert rel_l2(a["out"][t], ora["out"]) <= 1e-3
 
 
-def test_q8_router_grouped_and_prefill(ctx):
-    # 48 fp32 tokens through the grouped experts (the per-token router kernel
-    # serves a non-bf16 router) and a bf16 prefill chunk (widened for it).
-    seed, D, I, G, E, k, T = 62, 512, 256, 64, 64, 6, 48
+# fp32 tokens through the grouped experts and a bf16 prefill chunk: 48 take the fp64 router GEMM, which reads either;
+# for 24 the per-token router kernel serves a router that is not bf16, and the prefill chunk is widened for it.
+@pytest.mark.parametrize("T", [48, 24])
+def test_q8_router_grouped_and_prefill(ctx, T):
+    seed, D, I, G, E, k = 62, 512, 256, 64, 64, 6
     g, slab, shared, q8, f32, r32, s32 = build(ctx, seed, D, I, G, E, k, 64, T)
     x = O.synth_tokens(seed, 100, T, D)
     for m in (q8, f32):
@@ -92,6 +93,7 @@ def test_q8_router_grouped_and_prefill(ctx):
     f32.set_path(osm_hip.PATH_PER_TOKEN)
     per = f32.run_slab(slab, 0, xw)
     assert rel_l2(got, per["out"].reshape(-1)) <= 2e-5
+    assert np.array_equal(q8.routing(T)["ids"], per["ids"])
 
 
 def test_q8_router_rejected_shapes(ctx):

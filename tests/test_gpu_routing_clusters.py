@@ -7,6 +7,7 @@ import pytest
 
 import oracle as O
 import osm_hip
+from helpers import bf16_bits
 from test_gpu_routing_exact import _libm_expf, _softmax_sum
 
 pytestmark = pytest.mark.gpu
@@ -69,15 +70,28 @@ def rows_for(logits):
     return router
 
 
-def every_selection(ctx, router, k, x, xin, nw):
-    """(label, ids, stats) of each kernel that selects for the router's input x (xin, normalised with nw): one token and four (inside gate/up), 16 (the selection kernel
-    behind the per-token router), 48 (behind the router GEMM), with and without the norm, and 1,024 bf16 tokens."""
+def encoded(router, kind):
+    """The layer's router arguments for a router of whole numbers from -5 to 250 (kinds but f32)."""
+    if kind == "f32":
+        return router, osm_hip.F32
+    if kind == "q8":  # value q - 5, groups of 32
+        q = (router + 5).astype(np.uint32)
+        packed = (q[:, 0::4] | (q[:, 1::4] << 8) | (q[:, 2::4] << 16) | (q[:, 3::4] << 24)).astype(np.uint32)
+        one = np.ones((len(router), router.shape[1] // 32), np.float32)
+        return (packed, one, -5 * one, 32), osm_hip.AFFINE_Q8
+    return (router.astype(np.float16), osm_hip.F16) if kind == "f16" else (bf16_bits(router), osm_hip.BF16)
+
+
+def every_selection(ctx, router, k, x, xin, nw, kind="f32"):
+    """(label, ids, stats) of each kernel that selects for the router's input x (xin, normalised with nw): one token and
+    four (inside gate/up), 16 (the selection kernel behind the per-token router), 48 (behind the router GEMM), with and
+    without the norm, and 1,024 bf16 tokens."""
     E, D = router.shape
     I, G = 128, 64
     g = osm_hip.geometry(D, I, G, osm_hip.BF16)
     slab = osm_hip.ExpertSlab(ctx, g, 1, E)
     slab.synthesize(1)
-    moe = osm_hip.MoeLayer(ctx, g, E, k, router, osm_hip.F32, None, nw, None, max_tokens=1024, rms_eps=1e-20)
+    moe = osm_hip.MoeLayer(ctx, g, E, k, *encoded(router, kind), None, nw, None, max_tokens=1024, rms_eps=1e-20)
     assert np.array_equal(O.rms_norm(xin, 1, D, nw, 1e-20), x)
     for sublayer in (False, True):
         for T, path in ((1, osm_hip.PATH_PER_TOKEN), (4, osm_hip.PATH_PER_TOKEN), (16, osm_hip.PATH_PER_TOKEN),
@@ -182,3 +196,60 @@ def distance_rows(case):
 def test_distance_from_the_largest_logit(ctx, case, want):
     x = np.ones(EXACT_D, np.float32)
     assert check_rows(ctx, distance_rows(case), 2, x, x, 1.0) == want
+
+
+# Chains whose running value leaves their exact sum by tens (as above), from column `at` on, so that a chunk of 32 columns
+# starts from none of the values around its exact start and is run once more; their logits, in the opposite order to the
+# device's, decide the picks. 0: every chunk but the first; 20: across a boundary, where the value is a few units off, and
+# the rest; 200: the last chunk alone.
+@pytest.mark.parametrize("at", [0, 20, 200])
+def test_chunk_from_another_start(ctx, at):
+    router = np.zeros((40, EXACT_D), np.float32)
+    router[:, -1] = -2000
+    moved(router[33, at:], 20, 4, 3)  # 83 by the device's sums
+    moved(router[36, at:], 10, 4, 5)  # 45
+    x = np.ones(EXACT_D, np.float32)
+    want = O.route_qwen_top_k(x, router, EXACT_D, 40, 2, True)["ids"]
+    assert list(want) == [36, 33]
+    for label, ids, stats in every_selection(ctx, router, 2, x, x, x):
+        assert np.array_equal(ids, np.tile(want, (len(ids), 1))), (label, ids[0])
+        assert stats["exact"] == len(ids) and stats["exact_all"] == 0, (label, stats)
+
+
+# Logits a + b s for a first column of 1 and one of s near the end (past column 2,048 at hidden 4,096), the router's
+# values whole numbers that every dtype holds. 40 experts are two to a thread, 520 four.
+SHAPES = [(256, 40), (1024, 520), (4096, 520)]
+
+
+def two_columns(ctx, D, E, kind, k, s, logits):
+    router = np.zeros((E, D), np.float32)
+    router[:, 0] = -5
+    for e, (a, b) in logits.items():
+        router[e, 0], router[e, D - 2] = a, b
+    x = np.zeros(D, np.float32)
+    x[0], x[D - 2] = 1, s
+    root = np.float32(D**0.5)
+    want = O.route_qwen_top_k(x, router, D, E, k, True)["ids"]
+    for label, ids, stats in every_selection(ctx, router, k, x, root * x, np.full(D, 1 / root, np.float32), kind):
+        assert np.array_equal(ids, np.tile(want, (len(ids), 1))), (label, ids[0], want)
+        assert stats["exact"] == len(ids), (label, stats)
+        yield label, len(ids), stats, list(want)
+
+
+# Two clusters that the bounds leave open, one across the end of the picks, every logit apart by more than the tie margin:
+# no token needs the full recompute.
+@pytest.mark.parametrize("D,E", SHAPES)
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16", "q8"])
+def test_open_clusters_every_router(ctx, D, E, kind):
+    logits = {7: (8, 2), 30: (8, 0), 3: (8, 1), 12: (4, 0), 25: (4, 1)}
+    for label, tokens, stats, want in two_columns(ctx, D, E, kind, 4, 2.0**-17, logits):
+        assert want == [7, 3, 30, 25] and stats["exact_all"] == 0, (label, stats)
+
+
+# Every pick but the first more than 80 below the largest logit: every token needs it, and the second column decides.
+@pytest.mark.parametrize("D,E", SHAPES)
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16", "q8"])
+def test_full_recompute_every_router(ctx, D, E, kind):
+    logits = {0: (100, 0), 20: (15, 200), 30: (15, 100), 10: (15, 0)}
+    for label, tokens, stats, want in two_columns(ctx, D, E, kind, 3, 2.0**-13, logits):
+        assert want == [0, 20, 30] and stats["exact_all"] == tokens, (label, stats)
