@@ -51,6 +51,7 @@ constexpr uint32_t kGroupedWaves = 4;
 constexpr uint32_t kGroupedThreads = kGroupedWaves * kWave;
 constexpr uint32_t kRouterSplit = 3;
 constexpr uint32_t kRouterGemmMinTokens = 16;
+constexpr uint64_t kRouterF64MinProducts = 1u << 23;  // the fp64 router GEMM, bf16 input
 constexpr uint32_t kActSplit = 2;
 
 __device__ __forceinline__ uint16_t bf16_rne(float f) {
@@ -1550,10 +1551,25 @@ int osmd_moe_grouped(const osmd_moe_grouped_args* a, osmd_stream s) {
   // GEMMs: 3 bf16 terms per activation for the router, of which the expert
   // GEMMs read the first 2 (the group sums are of those 2).
   const bool router_gemm = m.router_dtype == OSM_META_BF16 && (xbf16 || T > kRouterGemmMinTokens);
-  // A router of another dtype runs as a GEMM in fp64 from the automatic
-  // path's 40 tokens on, reading x itself (one 512-token pass of an 8-bit
-  // router: 400 µs as per-token GEMVs, 48 µs).
+  // A router of another dtype runs as a GEMM in fp64, reading x itself, from
+  // the automatic path's 40 tokens on and where there is enough of it (one
+  // 512-token pass of a 512-expert 8-bit router: 400 µs as per-token GEMVs, 48
+  // µs). The GEMM takes some 10 µs however few its products are; the GEMV's
+  // time follows tokens x rows x columns, a row of up to 2,048 columns costing
+  // as much as one of them. Layers with experts of 128, fp32 input, µs with the
+  // GEMV / the GEMM for an fp32 router (8-bit and f16 routers alike but for the
+  // last): hidden 2,048, 8 experts, 40 tokens 48 / 56; 64 experts, 64 tokens
+  // (0.34 of the line) 69 / 76, 200 tokens (1.06) 94 / 91; hidden 512, 512
+  // experts, 40 tokens (1.7) 68 / 56; 8,192, 64 experts, 100 tokens (2.1) 157 /
+  // 139, 8 bits 157 / 155. A bf16 input has to be widened for the GEMV and
+  // gains from a third of that: hidden 2,048, 64 experts, 40 tokens (0.63 of
+  // its line) 64 / 63, 8 bits 57 / 59, f16 53 / 63; 100 tokens (1.6) 76 / 72,
+  // 78 / 76, 72 / 71.
+  const uint64_t router_products = static_cast<uint64_t>(T) *
+                                   (m.expert_count + ((m.flags & OSMD_MOE_SHARED) ? 1u : 0u)) *
+                                   (D < 2048u ? 2048u : D);
   const bool router_f64 = m.router_dtype != OSM_META_BF16 && T >= OSMD_GROUPED_MIN_TOKENS &&
+                          router_products >= (xbf16 ? 1u : 3u) * kRouterF64MinProducts &&
                           a->logit_planes64 != nullptr && a->router_norms != nullptr && a->x_norms != nullptr &&
                           a->bound_planes != nullptr;
   if (xbf16 && !router_gemm && !router_f64) {

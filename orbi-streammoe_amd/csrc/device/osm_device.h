@@ -263,11 +263,12 @@ typedef struct osmd_moe_grouped_args {
   float* x_norms;
   float* bound_planes;
   /* The logit planes of a router that is not bf16, in fp64, or null: such a
-   * router then runs as one GEMV per token and row. */
+   * router then runs as one GEMV per token and row, as it does for small
+   * routers and few tokens. */
   double* logit_planes64;
 } osmd_moe_grouped_args;
 /* Tokens from which a layer's decodes take the grouped path by themselves,
- * and from which a router that is not bf16 runs as a GEMM. */
+ * and from which a router that is not bf16 may run as a GEMM. */
 #define OSMD_GROUPED_MIN_TOKENS 40u
 /* Norms of a router's 32-column chunks, [E + 1][D/32] (row E only with a
  * shared gate), each rounded up; any dtype but bf16. */

@@ -71,9 +71,9 @@ def test_q8_router_decode_matches_fp32_and_oracle(ctx, group):
         assert rel_l2(a["out"][t], ora["out"]) <= 1e-3
 
 
-# fp32 tokens through the grouped experts and a bf16 prefill chunk: 48 take the fp64 router GEMM, which reads either;
-# for 24 the per-token router kernel serves a router that is not bf16, and the prefill chunk is widened for it.
-@pytest.mark.parametrize("T", [48, 24])
+# fp32 tokens through the grouped experts and a bf16 prefill chunk: 200 take the fp64 router GEMM, which reads either;
+# for 48 and 24 the per-token router kernel serves a router that is not bf16, and the prefill chunk is widened for it.
+@pytest.mark.parametrize("T", [48, 200, 24])
 def test_q8_router_grouped_and_prefill(ctx, T):
     seed, D, I, G, E, k = 62, 512, 256, 64, 64, 6
     g, slab, shared, q8, f32, r32, s32 = build(ctx, seed, D, I, G, E, k, 64, T)

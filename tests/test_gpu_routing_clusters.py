@@ -84,8 +84,9 @@ def encoded(router, kind):
 
 def every_selection(ctx, router, k, x, xin, nw, kind="f32"):
     """(label, ids, stats) of each kernel that selects for the router's input x (xin, normalised with nw): one token and
-    four (inside gate/up), 16 (the selection kernel behind the per-token router), 48 (behind the router GEMM), with and
-    without the norm, and 1,024 bf16 tokens."""
+    four (inside gate/up), 16 (the selection kernel behind the per-token router), 48 and 320 (grouped, behind the router
+    GEMM, of which routers that are not bf16 and of few rows take the second alone), with and without the norm, and 1,024
+    bf16 tokens."""
     E, D = router.shape
     I, G = 128, 64
     g = osm_hip.geometry(D, I, G, osm_hip.BF16)
@@ -95,7 +96,7 @@ def every_selection(ctx, router, k, x, xin, nw, kind="f32"):
     assert np.array_equal(O.rms_norm(xin, 1, D, nw, 1e-20), x)
     for sublayer in (False, True):
         for T, path in ((1, osm_hip.PATH_PER_TOKEN), (4, osm_hip.PATH_PER_TOKEN), (16, osm_hip.PATH_PER_TOKEN),
-                        (48, osm_hip.PATH_GROUPED)):
+                        (48, osm_hip.PATH_GROUPED), (320, osm_hip.PATH_GROUPED)):
             moe.set_path(path)
             xd, yd = ctx.alloc(T * D * 4), ctx.alloc(T * D * 4)
             xd.upload(np.tile(xin if sublayer else x, (T, 1)))
