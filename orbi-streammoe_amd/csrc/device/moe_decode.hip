@@ -1120,9 +1120,11 @@ __device__ bool resolve_clusters(const RouteView& rv, uint32_t t, Selection<PER>
 // alone (gate/up, whose selection every workgroup repeats and which wants three
 // wavefronts to a SIMD: 151 to 168 registers. With the clusters' code and
 // full_logits it takes 212 to 236, two wavefronts: 4 tokens' sublayers took 4%
-// longer; one token's took, hidden 2,048, top-10 and the shared expert, µs a
-// layer, plain / with clusters, 22.1 / 25.4 at intermediate 640, 23.6 / 26.8 at
-// 768, and 20.6 / 20.4 and 19.1 / 19.0 at 512 with 600 and 512 experts);
+// longer. One token's launch takes them where its workgroups fit the chip two
+// to a compute unit: hidden 2,048, top-10 and the shared expert, µs a layer,
+// plain / with clusters, intermediate 512 (473 workgroups) 20.0 / 19.7 in a step
+// with open tokens and 20.7 / 20.4 with 600 experts; 640 (594) 22.1 / 25.4 and
+// 768 (704) 23.6 / 26.8);
 // kExactClusters open clusters first, and the full recompute by
 // full_logits; kExactDeep the general form with its loads two steps ahead (246
 // to 255 registers: either of the other two beside it spills or halves the
@@ -1938,6 +1940,7 @@ __global__ __launch_bounds__(256) void route_kernel(osmd_moe_args a) {
 // at 4 and 16 tokens three rows measured 14% and 20% slower than eight.
 constexpr int kGuWaves = 4;
 constexpr int kGuRowsOneToken = 3;
+constexpr uint32_t kOneTokenClusterGroups = 512;  // two to each of 256 compute units (ExactMode)
 constexpr int kGuRowsBatched = 8;
 
 // Lane's slices of x (chunks lane, lane+64, ... of 32 floats). Lanes past the
@@ -2033,7 +2036,7 @@ __device__ __forceinline__ void gate_up_rows(const GateUpParams& p, uint32_t t, 
   }
 }
 
-template <int META, int CPL, int PER, int ROWS>
+template <int META, int CPL, int PER, int ROWS, ExactMode MODE = kExactPlain>
 __global__ __launch_bounds__(256) void gate_up_kernel(GateUpParams p) {
   const uint32_t t = blockIdx.z;
   const uint32_t j = blockIdx.y;
@@ -2055,7 +2058,7 @@ __global__ __launch_bounds__(256) void gate_up_kernel(GateUpParams p) {
       // forms the probabilities.
       const bool publisher = blockIdx.x == 0 && j == 0;
       OSMD_STAMP(4, timeline_first());
-      select_block<PER, false, kExactPlain>(rv, t, sel, false, publisher);
+      select_block<PER, false, MODE>(rv, t, sel, false, publisher);
       OSMD_STAMP(8, timeline_first());
       rows(pick_blob(rv, sel, j));
       OSMD_STAMP(10, timeline_first());
@@ -2530,23 +2533,34 @@ int pow2_at_least(uint32_t v) {
   return p;
 }
 
+// One token with the open-cluster form, for rows of one chunk per lane (hidden
+// up to 2,048: wider layers have no use for it).
+template <int META, int CPL, int PER>
+void launch_one_token_clusters(const GateUpParams& gp, dim3 grid, hipStream_t st) {
+  static_assert(64u * 32u == kSplitMaxCols, "CPL 1 is what the split chains take");
+  if constexpr (CPL == 1) gate_up_kernel<META, 1, PER, kGuRowsOneToken, kExactClusters><<<grid, 256, 0, st>>>(gp);
+}
+
 template <int META, int CPL>
 int launch_gate_up_cpl(const GateUpParams& gp, uint32_t tokens, int per, hipStream_t st) {
   const bool one = tokens == 1u;
   const uint32_t rows_per_block = kGuWaves * (one ? kGuRowsOneToken : kGuRowsBatched);
   const dim3 grid((gp.g.inter + rows_per_block - 1) / rows_per_block, gp.list.count ? gp.list.count : gp.src.nslot,
                   tokens);
+  const bool clusters = CPL == 1 && one && gp.g.hidden % 128u == 0u && grid.x * grid.y <= kOneTokenClusterGroups;
   switch (per) {
     case 0:
       if (one) gate_up_kernel<META, CPL, 0, kGuRowsOneToken><<<grid, 256, 0, st>>>(gp);
       else gate_up_kernel<META, CPL, 0, kGuRowsBatched><<<grid, 256, 0, st>>>(gp);
       break;
     case 2:
-      if (one) gate_up_kernel<META, CPL, 2, kGuRowsOneToken><<<grid, 256, 0, st>>>(gp);
+      if (clusters) launch_one_token_clusters<META, CPL, 2>(gp, grid, st);
+      else if (one) gate_up_kernel<META, CPL, 2, kGuRowsOneToken><<<grid, 256, 0, st>>>(gp);
       else gate_up_kernel<META, CPL, 2, kGuRowsBatched><<<grid, 256, 0, st>>>(gp);
       break;
     default:
-      if (one) gate_up_kernel<META, CPL, 4, kGuRowsOneToken><<<grid, 256, 0, st>>>(gp);
+      if (clusters) launch_one_token_clusters<META, CPL, 4>(gp, grid, st);
+      else if (one) gate_up_kernel<META, CPL, 4, kGuRowsOneToken><<<grid, 256, 0, st>>>(gp);
       else gate_up_kernel<META, CPL, 4, kGuRowsBatched><<<grid, 256, 0, st>>>(gp);
       break;
   }

@@ -15,11 +15,13 @@ pytestmark = pytest.mark.gpu
 
 # 128 columns: one run of 16 per chunk. 2,048: the widest of the split chains; 2,176 and 192 are left to the general
 # form, in the sublayer form too. Clusters of up to six open experts are settled apart, seven and eight go to the general
-# form. More than 512 experts: four to a thread.
-@pytest.mark.parametrize("D,E", [(128, 40), (192, 40), (1920, 40), (2048, 40), (2176, 40), (384, 520), (2176, 520)])
+# form. More than 512 experts: four to a thread. Intermediate 1,088: more than 512 workgroups for one token, which then
+# takes the general form too.
+@pytest.mark.parametrize("D,E,I", [(128, 40, 64), (192, 40, 64), (1920, 40, 64), (2048, 40, 64), (2176, 40, 64),
+                                   (384, 520, 64), (2176, 520, 64), (384, 40, 1088), (256, 520, 1088)])
 @pytest.mark.parametrize("clusters", [(2,), (3, 2), (6,), (7,), (2, 2, 2), (8, 3)])
-def test_routing_clusters(ctx, D, E, clusters):
-    I, G, k, T = 64, 64 if D % 64 == 0 else 32, 6, 24
+def test_routing_clusters(ctx, D, E, I, clusters):
+    G, k, T = 64 if D % 64 == 0 else 32, 6, 24
     seed = 5000 + D + sum(c * 10**i for i, c in enumerate(clusters))
     rng = np.random.default_rng(seed)
     g = osm_hip.geometry(D, I, G, osm_hip.BF16)
